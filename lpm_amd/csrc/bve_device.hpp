@@ -471,19 +471,26 @@ __device__ __forceinline__ void f64_block(const double4* __restrict__ src,
 // quads are summed from the start of each wave's run, a target's own source
 // is dropped by selects inside the same arithmetic, and the redone tiles
 // below are chosen per target.
-// 1 - x.y as one FMA chain from 1 leaves a residual of about 1e-17 where the
-// dot-then-subtract form gives exactly 0 (coincident points: a divided face
-// and its central child), so tiles with such a pair are redone in that form.
-// The screen is the high words of the products of two distances that the
-// shared reciprocal needs anyway (one three-way signed 32-bit minimum per
-// quad): such a distance is at most 4e-16 and its partner at most 2, so the
-// product is below kWaveRedo, or negative; two sources that are merely close
-// stay above it up to spacings of 3e-4.  (Screening the product of all four
-// flags nearly every free target of a refined cubed sphere of level 5: 78 us
-// against 60; screening each of the four 1 / d costs 2.6 % at level 5.)
+// 1 - x.y as one FMA chain from 1 is rounded otherwise than the pair formula's
+// 1 - (x.y): by about 1e-16, which at a distance d is 1e-16 / d of the pair's
+// term, and where the formula gives exactly 0 (coincident points: a divided
+// face and its central child) the chain leaves about 1e-17.  So tiles with a
+// distance below about 2^-20 are redone in the formula's order.  The screen:
+//  - of arbitrary points (MESH false): the high word of each distance, two
+//    three-way signed 32-bit minima per quad.  Free random points (12,345
+//    against 11,904 faces) then differ from the formula's sum by 1e-12 to
+//    2e-12, 0.2 % of their tiles redone; with 2^-24 1e-11 to 9e-11 and 0.02 %.
+//  - of the points of one mesh: the high words of the products of two distances
+//    that the shared reciprocal needs anyway, one minimum per quad (two cost
+//    3.3 % at level 7, 4.2 % at level 5), against 2^-36.  Neighbours in memory
+//    are neighbours in space there: a source that close has its sibling near,
+//    at 1e-5 at level 7, and the products of a level-8 mesh are above.  Where
+//    points come in any order that would miss a close source beside a distant
+//    one: with 2^-49 it left differences of up to 6e-7.
 constexpr int kQuadDoubles = 24;
 constexpr int kWaveTile = 16;  // quads per partial sum
-constexpr int kWaveRedo = 0x3CE00000;  // high word of 2^-49
+template <bool MESH>
+constexpr int kWaveRedo = MESH ? 0x3DB00000 : 0x3EB00000;  // 2^-36, 2^-20
 
 // Quads [*q0, *q1) of wave w of chunk `chunk` of C.
 __device__ __forceinline__ void wave_range(int nq, int chunk, int C, int w,
@@ -495,9 +502,8 @@ __device__ __forceinline__ void wave_range(int nq, int chunk, int C, int w,
 
 // Quads [qa, qb) into T.  CHECK drops each target's own source self[k] (its
 // distance is set to 1 and its weight to 0, leaving its neighbours' shared
-// reciprocal as it is).  low[k]: smallest high word of a product of two
-// distances.
-template <int TPL, bool EPS, bool CHECK>
+// reciprocal as it is).  low[k]: smallest high word of the screened values.
+template <int TPL, bool EPS, bool MESH, bool CHECK>
 __device__ __forceinline__ void wave_f64_quads(const double* __restrict__ quads,
                                                int qa, int qb,
                                                const double (*x)[3],
@@ -522,7 +528,12 @@ __device__ __forceinline__ void wave_f64_quads(const double* __restrict__ quads,
         if (CHECK && 4 * q + j == self[k]) d[j] = 1.0;
       }
       const double pab = d[0] * d[1], pcd = d[2] * d[3];
-      low[k] = min(low[k], min(__double2hiint(pab), __double2hiint(pcd)));
+      if (MESH) {
+        low[k] = min(low[k], min(__double2hiint(pab), __double2hiint(pcd)));
+      } else {
+        low[k] = min(low[k], min(__double2hiint(d[0]), __double2hiint(d[1])));
+        low[k] = min(low[k], min(__double2hiint(d[2]), __double2hiint(d[3])));
+      }
       const double r = rcp_nr<1>(pab * pcd);
       const double rab = r * pcd, rcd = r * pab;
       w[0] = d[1] * rab;
@@ -616,7 +627,7 @@ __device__ __forceinline__ int64_t lane_target(const SegArgs& sg, int64_t c,
 // sg.part[(3 c0 + comp) pstride + slot], else the chunk sums are added in
 // order and x cross S written.  Every thread of the 256 calls it; red holds
 // 4 x 64 TPL x 3 doubles.
-template <int TPL, bool EPS>
+template <int TPL, bool EPS, bool MESH>
 __device__ __forceinline__ void wave_f64_block(
     const double* __restrict__ quads, int nsrc, const SegArgs& sg, int blk,
     int c0, int c1, int C, double eps2, double (*red)[64 * TPL][3]) {
@@ -655,17 +666,19 @@ __device__ __forceinline__ void wave_f64_block(
 #pragma unroll
       for (int k = 0; k < TPL; ++k) low[k] = 0x7fffffff;
       if (lo < 4 * e && hi >= 4 * q)
-        wave_f64_quads<TPL, EPS, true>(quads, q, e, x, self, eps2, T, low);
+        wave_f64_quads<TPL, EPS, MESH, true>(quads, q, e, x, self, eps2, T,
+                                              low);
       else
-        wave_f64_quads<TPL, EPS, false>(quads, q, e, x, self, eps2, T, low);
+        wave_f64_quads<TPL, EPS, MESH, false>(quads, q, e, x, self, eps2, T,
+                                               low);
 #pragma unroll
       for (int k = 0; k < TPL; ++k)
-        if (__ballot(low[k] < kWaveRedo)) {
+        if (__ballot(low[k] < kWaveRedo<MESH>)) {
           double R[3];
           wave_f64_redo(quads, q, e, x[k], self[k], eps2, R);
 #pragma unroll
           for (int a = 0; a < 3; ++a)
-            T[k][a] = low[k] < kWaveRedo ? R[a] : T[k][a];
+            T[k][a] = low[k] < kWaveRedo<MESH> ? R[a] : T[k][a];
         }
 #pragma unroll
       for (int k = 0; k < TPL; ++k)

@@ -192,8 +192,9 @@ __global__ __launch_bounds__(256) void ens_wave_f64_kernel(
   const EnsMember M = A.mem[w.x];
   SegArgs sg = ens_segment(A, M, w.y);
   if (part) ens_parts(sg, M, w.y, part);
-  wave_f64_block<TPL, false>(quads + static_cast<int64_t>(M.P) * 6, M.cnt, sg, w.z,
-                      c0, part ? c0 + 1 : M.C, M.C, 0.0, red);
+  wave_f64_block<TPL, false, true>(quads + static_cast<int64_t>(M.P) * 6, M.cnt,
+                                   sg, w.z, c0, part ? c0 + 1 : M.C, M.C, 0.0,
+                                   red);
 }
 
 // Adds the chunk partials of the PER targets of each work item, one block per

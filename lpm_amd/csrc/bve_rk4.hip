@@ -373,6 +373,7 @@ void velocity_segments(lpm_ctx* ctx, const lpm_bve_fields& f, CrdIn vx,
   segs[1] = face_targets(fx, map, f.face_mask,
                          (flags & LPM_FLAG_SKIP_MASKED_TARGETS) != 0,
                          CrdOut{f.face_u, f.face_u_es, f.face_u_cs}, nullptr);
+  segs[0].mesh = segs[1].mesh = true;
 }
 
 void velocity_eval(lpm_ctx* ctx, const lpm_bve_fields& f, CrdIn vx, CrdIn fx,

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(BLOCK) void bve_vel_f64_split_kernel(
 
 // Wave-split sums (wave_f64_block): with partial sums (s0.part), block
 // b * C + k sums chunk k of target block b; without, block b sums every chunk.
-template <int TPL, bool EPS>
+template <int TPL, bool EPS, bool MESH>
 __global__ __launch_bounds__(256) void bve_wave_f64_kernel(
     const double* __restrict__ quads, const int32_t* __restrict__ count,
     SegArgs s0, SegArgs s1, double eps2, int C) {
@@ -305,8 +305,8 @@ __global__ __launch_bounds__(256) void bve_wave_f64_kernel(
   const bool first = b < s0.nblocks;
   const SegArgs& sg = pick(s0, s1, first);
   const int blk = first ? b : b - s0.nblocks;
-  wave_f64_block<TPL, EPS>(quads, *count, sg, blk, c0, split ? c0 + 1 : C, C, eps2,
-                      red);
+  wave_f64_block<TPL, EPS, MESH>(quads, *count, sg, blk, c0, split ? c0 + 1 : C,
+                                 C, eps2, red);
 }
 
 __global__ __launch_bounds__(256) void bve_wave_reduce_kernel(SegArgs s0,
@@ -1098,10 +1098,15 @@ void launch_wave_f64(lpm_ctx* ctx, const PackedSources& src,
   }
   const dim3 grid(static_cast<unsigned>(a0.nblocks + a1.nblocks) *
                   (split ? C : 1));
-  const auto kernel = tpl == 2 ? (eps2 > 0 ? bve_wave_f64_kernel<2, true>
-                                           : bve_wave_f64_kernel<2, false>)
-                               : (eps2 > 0 ? bve_wave_f64_kernel<1, true>
-                                           : bve_wave_f64_kernel<1, false>);
+  const bool mesh = t0.mesh && (t1.n == 0 || t1.mesh);
+  const auto pick_kernel = [&](auto t) {
+    constexpr int T = decltype(t)::value;
+    return eps2 > 0 ? bve_wave_f64_kernel<T, true, false>
+           : mesh   ? bve_wave_f64_kernel<T, false, true>
+                    : bve_wave_f64_kernel<T, false, false>;
+  };
+  const auto kernel = tpl == 2 ? pick_kernel(std::integral_constant<int, 2>{})
+                               : pick_kernel(std::integral_constant<int, 1>{});
   hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, src.quad, src.count, a0,
                      a1, eps2, C);
   LPM_HIP_CHECK(hipGetLastError());

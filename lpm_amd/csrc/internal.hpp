@@ -91,6 +91,8 @@ struct TargetSeg {
                                        // i's own source, < 0 if none
   bool self_identity = false;          // collocated: self = slot c
   const uint8_t* skip = nullptr;       // targets to leave untouched
+  bool mesh = false;                   // points of the sources' mesh, in its
+                                       // order (else: arbitrary points)
   CrdOut out{nullptr, 0, 0};           // velocity output
   double* out_scalar = nullptr;        // stream-function output
 };
