@@ -67,6 +67,15 @@ __device__ __forceinline__ double rcp_nr(double d) {
   return r;
 }
 
+// The same by one third-order step, r <- r + r (e + e^2) with e = 1 - d r: the
+// estimate's 4.6e-8 cubed is far below a rounding, as after two Newton steps,
+// for three operations instead of four.
+__device__ __forceinline__ double rcp_cubic(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = __builtin_fma(-d, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+
 // FP64 natural logarithm of a distance, table-driven after P. T. P. Tang,
 // "Table-driven implementation of the logarithm function in IEEE
 // floating-point arithmetic", ACM TOMS 16(4), 1990.  With a = m 2^e, m in
@@ -462,10 +471,11 @@ __device__ __forceinline__ void f64_block(const double4* __restrict__ src,
 // LDS reads cost 32 cycles of a CU's LDS per source and wave, which bounds
 // fewer than four targets per lane; scalar loads leave one target per lane
 // as fast as four, so small problems fill the chip.
-// What bounds it: FP64 issue, 8.25 operations and a quarter reciprocal per
-// pair.  Level 7 (491,522 x 327,680 pairs, random points): 44.3 ms = 3,640
-// Gpairs/s, against 48.5-50 ms for the best LDS-staged split shape and 70 ms
-// for block256_tpl2_nr2_pairtrue; 7,682 x 5,120 pairs 17 us (about 250 us).
+// What bounds it: FP64 issue, 8.5 operations and a quarter reciprocal per
+// pair.  Level 7 (491,522 x 327,680 pairs): 45.4 ms = 3,550 Gpairs/s, 2.4 % more
+// than with one Newton step in the reciprocal, against 48.5-50 ms for the best
+// LDS-staged split shape (of one Newton step) and 70 ms for
+// block256_tpl2_nr2_pairtrue; 7,682 x 5,120 pairs 17 us (about 250 us).
 // The sums do not depend on TPL or on how many chunks a block takes: chunk
 // boundaries follow from C and the source count alone, tiles of up to 16
 // quads are summed from the start of each wave's run, a target's own source
@@ -534,7 +544,7 @@ __device__ __forceinline__ void wave_f64_quads(const double* __restrict__ quads,
         low[k] = min(low[k], min(__double2hiint(d[0]), __double2hiint(d[1])));
         low[k] = min(low[k], min(__double2hiint(d[2]), __double2hiint(d[3])));
       }
-      const double r = rcp_nr<1>(pab * pcd);
+      const double r = rcp_cubic(pab * pcd);
       const double rab = r * pcd, rcd = r * pab;
       w[0] = d[1] * rab;
       w[1] = d[0] * rab;

@@ -716,7 +716,7 @@ constexpr int kNumF64 = sizeof(kF64Variants) / sizeof(kF64Variants[0]);
 constexpr int kNumMixed = sizeof(kMixedVariants) / sizeof(kMixedVariants[0]);
 // Variants used until the autotuner (or the caller) picks another one.  The
 // wave-split kernel is the fastest FP64 shape from 2e6 pairs (L3: 8 us
-// against 93 us for variant 1) to 1.6e11 (44 ms; variant 25 48.5, variant 1
+// against 93 us for variant 1) to 1.6e11 (45 ms; variant 25 48.5, variant 1
 // 70).  The others keep their numbers: saved tuning tables hold them.
 constexpr int kDefaultF64 = 26;
 // The mixed default is the matrix-core kernel: 1.45 ms per level-6 evaluation

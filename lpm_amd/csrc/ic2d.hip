@@ -63,7 +63,7 @@ __device__ __forceinline__ void ic2d_quads(const double* __restrict__ rec,
       top = max(top, log_screen(d[j]));
     }
     const double pab = d[0] * d[1], pcd = d[2] * d[3];
-    const double r = rcp_nr<1>(pab * pcd);
+    const double r = rcp_cubic(pab * pcd);
     const double rab = r * pcd, rcd = r * pab;
     w[0] = d[1] * rab;
     w[1] = d[0] * rab;
