@@ -26,7 +26,9 @@
  *    different stream than the context's previous call, the library orders
  *    it after the previous stream's work (an event wait, no host sync).  A
  *    call on a stream that is being captured by the caller is not ordered
- *    this way: order such streams yourself.
+ *    this way: order such streams yourself.  Workspaces that such a call has
+ *    recorded stay allocated until the context is destroyed, also when later
+ *    calls outgrow them, so the caller's graph can be replayed that long.
  *  - Sums whose target blocks would leave the device underfilled split each
  *    block's sources into chunks and add the chunk partials in a second
  *    kernel (the stream function and Incompressible2D sums always when

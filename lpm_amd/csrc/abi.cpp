@@ -54,10 +54,12 @@ void set_error(lpm_ctx* ctx, const std::string& msg) {
 hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
 void order_stream(lpm_ctx* ctx, hipStream_t s) {
-  if (ctx->has_last_stream && ctx->last_stream == s) return;
+  const bool same = ctx->has_last_stream && ctx->last_stream == s;
+  if (same && !s) return;  // the null stream is never captured
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   LPM_HIP_CHECK(hipStreamIsCapturing(s, &st));
-  if (st != hipStreamCaptureStatusNone) return;
+  ctx->kept.call(st != hipStreamCaptureStatusNone);
+  if (same || st != hipStreamCaptureStatusNone) return;
   if (ctx->has_last_stream) {
     if (!ctx->order_event)
       LPM_HIP_CHECK(hipEventCreateWithFlags(&ctx->order_event,
@@ -71,17 +73,26 @@ void order_stream(lpm_ctx* ctx, hipStream_t s) {
 
 std::atomic<uint64_t> g_workspace_epoch{0};
 
-DevBuf::~DevBuf() {
-  if (ptr) (void)hipFree(ptr);
+KeptMemory::~KeptMemory() {
+  for (void* p : ptrs) (void)hipFree(p);
 }
+
+hipError_t DevBuf::release() {
+  if (!ptr) return hipSuccess;
+  void* p = ptr;
+  ptr = nullptr;
+  bytes = 0;
+  g_workspace_epoch.fetch_add(1);
+  if (!kept || !kept->recorded(born)) return hipFree(p);
+  kept->ptrs.push_back(p);
+  return hipSuccess;
+}
+
+DevBuf::~DevBuf() { (void)release(); }
 
 void* DevBuf::ensure(size_t nbytes) {
   if (nbytes <= bytes && ptr) return ptr;
-  if (ptr) {
-    LPM_HIP_CHECK(hipFree(ptr));
-    ptr = nullptr;
-    bytes = 0;
-  }
+  LPM_HIP_CHECK(release());
   const size_t want = std::max<size_t>(nbytes, 256);
   hipError_t e = hipMalloc(&ptr, want);
   if (e != hipSuccess) {
@@ -91,6 +102,7 @@ void* DevBuf::ensure(size_t nbytes) {
                                    " bytes failed: " + hipGetErrorString(e));
   }
   bytes = want;
+  born = kept ? kept->serial : 0;
   g_workspace_epoch.fetch_add(1);
   return ptr;
 }

@@ -141,6 +141,7 @@ std::shared_ptr<lpm_ctx::EnsemblePlan> plan_for(lpm_ctx* ctx,
                 "too many work items");
   np->n_items = static_cast<int>(w.size());
   np->n_chunk_items = static_cast<int>(wc.size());
+  np->members.kept = np->items.kept = np->chunk_items.kept = &ctx->kept;
   void* dm = np->members.ensure(sizeof(EnsMember) * M);
   void* di = np->items.ensure(sizeof(int4) * std::max<size_t>(w.size(), 1));
   LPM_HIP_CHECK(hipMemcpy(dm, mem.data(), sizeof(EnsMember) * M,

@@ -36,20 +36,39 @@ struct Error : std::runtime_error {
     if (!(cond)) throw ::lpm_amd::Error(LPM_ERR_ARG, (msg));      \
   } while (0)
 
-// Incremented whenever any workspace is (re)allocated; captured graphs
+// Incremented whenever any workspace is allocated or given up; captured graphs
 // record it and are re-captured when it changed, so that a replay never
 // touches freed workspace memory.
 extern std::atomic<uint64_t> g_workspace_epoch;
+
+// Memory that a graph of the caller may still use: a call recorded by the
+// caller's own capture leaves the addresses of the context's buffers in a graph
+// that the library never sees.  So an outgrown buffer that such a call may have
+// recorded is kept until the context ends.
+struct KeptMemory {
+  uint64_t serial = 0;  // odd during a recorded call, of its own for each
+  std::vector<void*> ptrs;
+  ~KeptMemory();
+  void call(bool captured) {
+    if ((serial & 1) != captured) ++serial;
+    else if (captured) serial += 2;
+  }
+  // of a buffer allocated at serial `born`
+  bool recorded(uint64_t born) const { return (born & 1) || serial > born; }
+};
 
 // Grow-only device buffer owned by a context.
 struct DevBuf {
   void* ptr = nullptr;
   size_t bytes = 0;
+  KeptMemory* kept = nullptr;  // its context's (null: never recorded)
+  uint64_t born = 0;           // kept->serial when allocated
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf();
   void* ensure(size_t nbytes);  // reallocates (contents lost) when too small
+  hipError_t release();         // frees or keeps the memory
   template <typename T>
   T* as() const {
     return static_cast<T*>(ptr);
@@ -153,6 +172,8 @@ struct lpm_ctx {
   int num_cus = 0;
   std::string arch;
 
+  lpm_amd::KeptMemory kept;  // before the buffers, which end first
+
   // prologue workspaces
   lpm_amd::DevBuf rank;         // int32 per stored face
   lpm_amd::DevBuf inv;          // int32 per stored face (packed -> face)
@@ -221,6 +242,16 @@ struct lpm_ctx {
   };
   std::vector<std::unique_ptr<TargetOrder>> orders;
   uint64_t order_clock = 0;
+
+  lpm_ctx() {
+    for (lpm_amd::DevBuf* b :
+         {&rank, &inv, &block_counts, &packed64, &packed64sy, &quad,
+          &log_table, &split_part, &packed32, &centers, &mf_y, &mf_q, &mf_s,
+          &mf_t, &mf_c, &mf_a, &mf_t32, &mf_is, &mf_g, &flag, &diag,
+          &count_ident, &swe_packed, &swe_bounds, &swe_feat, &swe_far,
+          &ens_queue, &rk_v, &rk_f, &swe_v, &swe_f, &ic2d_v, &ic2d_f})
+      b->kept = &kept;
+  }
 };
 
 namespace lpm_amd {
@@ -229,7 +260,9 @@ void set_error(lpm_ctx* ctx, const std::string& msg);
 
 // Orders this call's work on stream s after everything the context issued
 // on the stream of its previous call (the workspaces are shared by all of
-// a context's calls).  No-op when the stream is unchanged or capturing.
+// a context's calls).  No-op when the stream is unchanged or capturing; a
+// capture is the caller's (the steps begin theirs later) and is counted in
+// ctx->kept.
 void order_stream(lpm_ctx* ctx, hipStream_t s);
 
 // Kernel variants of a family (KID_*) and the autotuning table.

@@ -84,6 +84,7 @@ const int32_t* target_order(lpm_ctx* ctx, CrdIn x, int64_t n,
   e->n = n;
   e->ranges = h;
   e->last_use = ++ctx->order_clock;
+  e->perm.kept = &ctx->kept;
   int32_t* d = static_cast<int32_t*>(e->perm.ensure(sizeof(int32_t) * n));
   LPM_HIP_CHECK(hipMemcpy(d, perm.data(), sizeof(int32_t) * n,
                           hipMemcpyHostToDevice));
