@@ -435,7 +435,7 @@ uint64_t ensemble_prepare(lpm_ctx* ctx, const EnsembleDesc& d,
   const EnsLayout L = ensemble_plan(ctx, d, v.block * v.tpl, v.chunks());
   ensure_sources(ctx, d, precision, v.wave);
   if (v.wave || v.chunked)
-    split_workspace(ctx, sizeof(double) * 3 * L.parts, s);
+    chunk_workspace(ctx, sizeof(double) * 3 * L.parts, s);
   if (precision == LPM_MIXED) bve_ens_vertex_order(ctx, d, f, s);
   return L.serial;
 }
@@ -499,7 +499,7 @@ void ensemble_velocity(lpm_ctx* ctx, const EnsembleDesc& d,
     constexpr int kTpl = 2;
     LPM_ARG_CHECK(v.block * v.tpl == 64 * kTpl, "wave-split item size");
     // no workspace (a caller's capture, no memory): whole items, same bits
-    double* part = split_workspace(ctx, sizeof(double) * 3 * L.parts, s);
+    double* part = chunk_workspace(ctx, sizeof(double) * 3 * L.parts, s);
     EnsArgs B = A;
     if (part) B.items = L.chunk_items;
     TimedLaunch tl(ctx, family, s, L.pairs);
@@ -545,7 +545,7 @@ void ensemble_velocity(lpm_ctx* ctx, const EnsembleDesc& d,
   }
   if (v.chunked) {
     // no workspace (a caller's capture, no memory): whole items, same bits
-    double* part = split_workspace(ctx, sizeof(double) * 3 * L.parts, s);
+    double* part = chunk_workspace(ctx, sizeof(double) * 3 * L.parts, s);
     EnsArgs B = A;
     if (part) B.items = L.chunk_items;
     TimedLaunch tl(ctx, family, s, L.pairs);

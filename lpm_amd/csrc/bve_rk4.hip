@@ -398,7 +398,7 @@ bool issue_chunk_step(lpm_ctx* ctx, const lpm_bve_fields& f, double dt,
   const int variant = bve_velocity_variant(ctx, precision, nt);
   if (!bve_variant_chunked(precision, variant)) return false;
   const size_t bytes = bve_split_bytes(precision, variant, nt, f.n_faces);
-  double* part = bytes ? split_workspace(ctx, bytes, s) : nullptr;
+  double* part = bytes ? chunk_workspace(ctx, bytes, s) : nullptr;
   if (!part) return false;
   const RankMap map = build_rank(ctx, f.face_mask, f.n_faces, s);
   const unsigned layouts = bve_variant_layouts(precision, variant);
@@ -747,7 +747,9 @@ int lpm_bve_rk4_step(lpm_ctx* ctx, const lpm_bve_fields* f, double dt,
       if (precision == LPM_MIXED)
         target_order(ctx, vert_crd(*f), f->n_verts, nullptr, 1, s);
       const size_t part = bve_split_bytes(precision, variant, nt, f->n_faces);
-      if (part) split_workspace(ctx, part, s);  // nullptr: runs unsplit
+      if (part)  // nullptr: runs unsplit
+        (bve_variant_chunked(precision, variant) ? chunk_workspace
+                                                 : split_workspace)(ctx, part, s);
       return 0;
     };
     run_step(ctx, *f, dt, Omega, precision, flags, s, true, prepare,

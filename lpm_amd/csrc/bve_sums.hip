@@ -1067,6 +1067,10 @@ double* split_workspace(lpm_ctx* ctx, size_t need, hipStream_t s) {
   }
 }
 
+double* chunk_workspace(lpm_ctx* ctx, size_t need, hipStream_t s) {
+  return need <= kChunkBytes ? split_workspace(ctx, need, s) : nullptr;
+}
+
 namespace {
 
 void launch_split_reduce(const SegArgs& a0, const SegArgs& a1, int ks,
@@ -1196,7 +1200,7 @@ void launch_bve_velocity(lpm_ctx* ctx, const PackedSources& src,
     const size_t need =
         bve_split_bytes(precision, variant, t0.n + t1.n, src.capacity);
     if (!part && timed && need) {
-      part = split_workspace(ctx, need, s);
+      part = chunk_workspace(ctx, need, s);
       part_bytes = part ? need : 0;
     }
     const bool f64 = precision == LPM_FP64;
@@ -1290,7 +1294,7 @@ void launch_bve_stream_fn(lpm_ctx* ctx, const PackedSources& src,
   const int C = log_chunks(nt, src.capacity);
   // one chunk, or no workspace (a caller's capture, no memory): whole blocks
   double* part =
-      C > 1 ? split_workspace(ctx, sizeof(double) * static_cast<size_t>(C) * nt,
+      C > 1 ? chunk_workspace(ctx, sizeof(double) * static_cast<size_t>(C) * nt,
                               s)
             : nullptr;
   if (part) {

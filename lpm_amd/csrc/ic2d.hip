@@ -398,7 +398,7 @@ void launch_ic2d(lpm_ctx* ctx, const PackedSources& src, TargetSeg* segs,
   const int ks = ic2d_chunks(precision, t0.n + t1.n, src.capacity);
   // no workspace (a caller's capture, no memory): whole blocks, chunk by chunk
   double* part =
-      ks > 1 ? split_workspace(ctx, ic2d_split_bytes(ks, t0.n + t1.n), s)
+      ks > 1 ? chunk_workspace(ctx, ic2d_split_bytes(ks, t0.n + t1.n), s)
              : nullptr;
   if (part) {
     a0.part = part;
@@ -646,7 +646,7 @@ int lpm_ic2d_rk2_step(lpm_ctx* ctx, const lpm_ic2d_fields* f, double dt,
           const int ks =
               ic2d_chunks(precision, f->n_verts + f->n_faces, f->n_faces);
           if (ks > 1)
-            split_workspace(ctx, ic2d_split_bytes(ks, f->n_verts + f->n_faces),
+            chunk_workspace(ctx, ic2d_split_bytes(ks, f->n_verts + f->n_faces),
                             s);
           return ic2d_key(*f, dt, Omega, eps, precision, flags, s);
         },

@@ -444,6 +444,17 @@ size_t bve_split_bytes(int precision, int variant, int64_t n_targets,
 // cannot be: s is capturing and it is smaller, or the device is out of
 // memory (the caller then runs an unsplit variant).
 double* split_workspace(lpm_ctx* ctx, size_t need, hipStream_t s);
+// The same for the sums in chunks by size, which also run without it, in whole
+// blocks to the same bits: nullptr above kChunkBytes.  They keep up to 24 C
+// (velocity), 8 C (stream function), 32 C (Incompressible2D) or 160 C
+// (shallow water) bytes a target, C from 8 on, so a bound is needed: FP64
+// shallow water of 1e7 targets would hold 12.8 GB.  At the bound, 2.8 million
+// targets in FP64 velocity and 839,000 in shallow water, the target blocks
+// alone fill the device many times.  Whole blocks against chunks: level 5
+// 1.3 to 3.9 times as long, level 6 1.08 to 1.6, level 7 (491,522 targets, 189
+// and 629 MB) 1.02 to 1.17; 1e6 and more targets 0.84 to 1.14.
+constexpr size_t kChunkBytes = size_t(1) << 30;
+double* chunk_workspace(lpm_ctx* ctx, size_t need, hipStream_t s);
 // Uploads the table of the FP64 logarithm (context creation).
 void make_log_table(lpm_ctx* ctx);
 void launch_bve_stream_fn(lpm_ctx* ctx, const PackedSources& src,

@@ -1911,6 +1911,12 @@ size_t swe_part_bytes(const SweVariant& v, int64_t n_targets, int64_t n_src) {
                     : kSweMfRows * swe_mf_chunks(n_targets, n_src));
 }
 
+// Far sums of whole blocks: one set per target.
+double* swe_far_rows(lpm_ctx* ctx, int64_t n_targets) {
+  return static_cast<double*>(ctx->swe_far.ensure(
+      sizeof(double) * kSweMfRows * std::max<int64_t>(n_targets, 1)));
+}
+
 SweSeg to_seg(const SweTargets& t, int per_block) {
   SweSeg a{};
   a.x = t.base.x.base;
@@ -1952,8 +1958,6 @@ void swe_feature_workspace(lpm_ctx* ctx, int64_t n_src, int64_t n_targets,
   if (!v.mf()) return;
   const int64_t ntile = (std::max<int64_t>(n_src, 1) + kSweTile - 1) / kSweTile;
   ctx->swe_feat.ensure(kSweMfTileBytes * ntile);
-  ctx->swe_far.ensure(sizeof(double) * kSweMfRows *
-                      std::max<int64_t>(n_targets, 1));
 }
 
 SweBounds swe_bounds(lpm_ctx* ctx, int precision, int64_t n_targets) {
@@ -1972,8 +1976,12 @@ void swe_sums_workspace(lpm_ctx* ctx, int64_t n_src, int64_t n_targets,
                         int precision, hipStream_t s) {
   swe_feature_workspace(ctx, n_src, n_targets, precision);
   const SweVariant& v = swe_variant(ctx, precision, n_targets);
-  if (v.wave || v.mf())
-    split_workspace(ctx, swe_part_bytes(v, n_targets, n_src), s);
+  if (!v.wave && !v.mf()) return;
+  const bool chunks = v.wave || swe_mf_chunks(n_targets, n_src) > 1;
+  const double* part =
+      chunks ? chunk_workspace(ctx, swe_part_bytes(v, n_targets, n_src), s)
+             : nullptr;
+  if (v.mf() && !part) swe_far_rows(ctx, n_targets);
 }
 
 SwePacked swe_pack_sources(lpm_ctx* ctx, CrdIn sx, const double* zeta,
@@ -2031,7 +2039,7 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
     const int C = swe_chunks(nt, src.capacity);
     // one chunk, or no workspace (a caller's capture, no memory): whole blocks
     double* part =
-        C > 1 ? split_workspace(ctx, swe_part_bytes(v, nt, src.capacity), s)
+        C > 1 ? chunk_workspace(ctx, swe_part_bytes(v, nt, src.capacity), s)
               : nullptr;
     a0.part = part;
     a1.part = part + (part ? kSweRows * static_cast<int64_t>(C) * a0.n : 0);
@@ -2059,13 +2067,11 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
     LPM_HIP_CHECK(hipGetLastError());
     P.C = swe_mf_chunks(nt, src.capacity);
     // one chunk, or no workspace (a caller's capture, no memory): whole blocks
-    double* far = static_cast<double*>(
-        ctx->swe_far.ensure(sizeof(double) * kSweMfRows * nt));
     double* part =
-        P.C > 1 ? split_workspace(ctx, swe_part_bytes(v, nt, src.capacity), s)
+        P.C > 1 ? chunk_workspace(ctx, swe_part_bytes(v, nt, src.capacity), s)
                 : nullptr;
     P.rows = part ? P.C : 1;
-    a0.part = part ? part : far;
+    a0.part = part ? part : swe_far_rows(ctx, nt);
     a1.part = a0.part + kSweMfRows * static_cast<int64_t>(P.rows) * a0.n;
     TimedLaunch tl(ctx, KID_SWE_MIXED, s, pairs);
     hipLaunchKernelGGL(v.far, dim3(static_cast<unsigned>(grid) * P.rows),
@@ -2104,12 +2110,11 @@ uint64_t swe_ensemble_prepare(lpm_ctx* ctx, const EnsembleDesc& d,
   const int64_t cap = std::max<int64_t>(d.total_padded_upper, kSweTile);
   ctx->swe_packed.ensure(sizeof(SweSrc) * cap);
   ctx->swe_bounds.ensure(sizeof(double4) * 5 * (cap / kSweTile));
-  if (v.wave) split_workspace(ctx, sizeof(double) * kSweRows * L.parts, s);
+  if (v.wave) chunk_workspace(ctx, sizeof(double) * kSweRows * L.parts, s);
   if (v.mf()) {
     ctx->swe_feat.ensure(kSweMfTileBytes * (cap / kSweTile));
-    ctx->swe_far.ensure(sizeof(double) * kSweMfRows *
-                        std::max<int64_t>(d.n_verts + d.n_faces, 1));
-    split_workspace(ctx, sizeof(double) * kSweMfRows * L.parts, s);
+    if (!chunk_workspace(ctx, sizeof(double) * kSweMfRows * L.parts, s))
+      swe_far_rows(ctx, d.n_verts + d.n_faces);
   }
   if (precision == LPM_MIXED) {
     swe_ens_vertex_order(ctx, d, f, s);
@@ -2175,7 +2180,7 @@ void swe_ensemble_sums(lpm_ctx* ctx, const EnsembleDesc& d,
                   eps == 0.0 ? 1 : 0};
   if (v.wave) {
     double* part =
-        split_workspace(ctx, sizeof(double) * kSweRows * L.parts, s);
+        chunk_workspace(ctx, sizeof(double) * kSweRows * L.parts, s);
     SweEnsArgs B = A;
     if (part) B.items = L.chunk_items;
     TimedLaunch tl(ctx, KID_SWE_F64, s, L.pairs);
@@ -2197,11 +2202,11 @@ void swe_ensemble_sums(lpm_ctx* ctx, const EnsembleDesc& d,
     swe_ens_mf_pack_kernel<<<grid2, 256, 0, s>>>(src, L.mem, A.P.mf);
     LPM_HIP_CHECK(hipGetLastError());
     double* part =
-        split_workspace(ctx, sizeof(double) * kSweMfRows * L.parts, s);
+        chunk_workspace(ctx, sizeof(double) * kSweMfRows * L.parts, s);
     A.P.rows = part ? 0 : 1;  // 0: each member's chunks
     SweEnsArgs B = A;
     if (part) B.items = L.chunk_items;
-    else part = ctx->swe_far.as<double>();
+    else part = swe_far_rows(ctx, d.n_verts + d.n_faces);
     TimedLaunch tl(ctx, KID_SWE_MIXED, s, L.pairs);
     hipLaunchKernelGGL(v.ens_far,
                        dim3(A.P.rows == 1 ? L.n_items : L.n_chunk_items),
