@@ -187,7 +187,8 @@ template <int TPL>
 __global__ __launch_bounds__(256) void ens_wave_f64_kernel(
     const double* __restrict__ quads, EnsArgs A, double* part) {
   __shared__ double red[4][64 * TPL][3];
-  const int4 w = A.items[blockIdx.x];
+  if (flat_block() >= A.n_items) return;
+  const int4 w = A.items[flat_block()];
   const int c0 = w.w;
   const EnsMember M = A.mem[w.x];
   SegArgs sg = ens_segment(A, M, w.y);
@@ -202,7 +203,8 @@ __global__ __launch_bounds__(256) void ens_wave_f64_kernel(
 template <int PER>
 __global__ __launch_bounds__(PER) void ens_chunk_reduce_kernel(EnsArgs A,
                                                                double* part) {
-  const int4 w = A.items[blockIdx.x];
+  if (flat_block() >= A.n_items) return;
+  const int4 w = A.items[flat_block()];
   const EnsMember M = A.mem[w.x];
   SegArgs sg = ens_segment(A, M, w.y);
   ens_parts(sg, M, w.y, part);
@@ -214,7 +216,8 @@ __global__ __launch_bounds__(256, 5) void ens_mfma16_chunk_kernel(
     Mfma16Src src, EnsArgs A, double* part) {
   __shared__ uint4 la[2 * kPackTile];
   __shared__ float4 lt[kPackTile];
-  const int4 w = A.items[blockIdx.x];
+  if (flat_block() >= A.n_items) return;
+  const int4 w = A.items[flat_block()];
   const EnsMember M = A.mem[w.x];
   SegArgs sg = ens_segment(A, M, w.y);
   if (part) ens_parts(sg, M, w.y, part);
@@ -501,10 +504,13 @@ void ensemble_velocity(lpm_ctx* ctx, const EnsembleDesc& d,
     // no workspace (a caller's capture, no memory): whole items, same bits
     double* part = chunk_workspace(ctx, sizeof(double) * 3 * L.parts, s);
     EnsArgs B = A;
-    if (part) B.items = L.chunk_items;
+    if (part) {
+      B.items = L.chunk_items;
+      B.n_items = L.n_chunk_items;
+    }
     TimedLaunch tl(ctx, family, s, L.pairs);
     ens_wave_f64_kernel<kTpl>
-        <<<part ? L.n_chunk_items : L.n_items, 256, 0, s>>>(
+        <<<launch_grid(B.n_items, 256), 256, 0, s>>>(
             ctx->quad.as<double>(), B, part);
     LPM_HIP_CHECK(hipGetLastError());
     if (part) {
@@ -547,9 +553,12 @@ void ensemble_velocity(lpm_ctx* ctx, const EnsembleDesc& d,
     // no workspace (a caller's capture, no memory): whole items, same bits
     double* part = chunk_workspace(ctx, sizeof(double) * 3 * L.parts, s);
     EnsArgs B = A;
-    if (part) B.items = L.chunk_items;
+    if (part) {
+      B.items = L.chunk_items;
+      B.n_items = L.n_chunk_items;
+    }
     TimedLaunch tl(ctx, family, s, L.pairs);
-    ens_mfma16_chunk_kernel<<<part ? L.n_chunk_items : L.n_items, 256, 0, s>>>(
+    ens_mfma16_chunk_kernel<<<launch_grid(B.n_items, 256), 256, 0, s>>>(
         ms16, B, part);
     LPM_HIP_CHECK(hipGetLastError());
     if (part) {

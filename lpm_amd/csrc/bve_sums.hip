@@ -300,8 +300,8 @@ __global__ __launch_bounds__(256) void bve_wave_f64_kernel(
     SegArgs s0, SegArgs s1, double eps2, int C) {
   __shared__ double red[4][64 * TPL][3];
   const bool split = s0.part != nullptr;
-  const int b = split ? static_cast<int>(blockIdx.x) / C : blockIdx.x;
-  const int c0 = split ? static_cast<int>(blockIdx.x) % C : 0;
+  const int b = split ? flat_block() / C : flat_block();
+  const int c0 = split ? flat_block() % C : 0;
   const bool first = b < s0.nblocks;
   const SegArgs& sg = pick(s0, s1, first);
   const int blk = first ? b : b - s0.nblocks;
@@ -403,8 +403,8 @@ __global__ __launch_bounds__(256, 5) void bve_vel_mfma16_chunk_kernel(
   __shared__ uint4 la[2 * kPackTile];
   __shared__ float4 lt[kPackTile];
   const bool split = s0.part != nullptr;
-  const int b = split ? static_cast<int>(blockIdx.x) / C : blockIdx.x;
-  const int c0 = split ? static_cast<int>(blockIdx.x) % C : 0;
+  const int b = split ? flat_block() / C : flat_block();
+  const int c0 = split ? flat_block() % C : 0;
   const bool first = b < s0.nblocks;
   const SegArgs& sg = pick(s0, s1, first);
   const int blk = first ? b : b - s0.nblocks;
@@ -474,8 +474,8 @@ __global__ __launch_bounds__(256) void bve_psi_kernel(
   __shared__ double2 ltab[kLogTable];
   __shared__ double red[4][64];
   const bool split = s0.part != nullptr;
-  const int b = split ? static_cast<int>(blockIdx.x) / C : blockIdx.x;
-  const int c0 = split ? static_cast<int>(blockIdx.x) % C : 0;
+  const int b = split ? flat_block() / C : flat_block();
+  const int c0 = split ? flat_block() % C : 0;
   const bool first = b < s0.nblocks;
   const SegArgs& sg = pick(s0, s1, first);
   const int blk = first ? b : b - s0.nblocks;
@@ -1100,8 +1100,8 @@ void launch_wave_f64(lpm_ctx* ctx, const PackedSources& src,
     a0.part = part;
     a1.part = part + 3 * static_cast<int64_t>(C) * t0.n;
   }
-  const dim3 grid(static_cast<unsigned>(a0.nblocks + a1.nblocks) *
-                  (split ? C : 1));
+  const dim3 grid = launch_grid(
+      (static_cast<int64_t>(a0.nblocks) + a1.nblocks) * (split ? C : 1), 256);
   const bool mesh = t0.mesh && (t1.n == 0 || t1.mesh);
   const auto pick_kernel = [&](auto t) {
     constexpr int T = decltype(t)::value;
@@ -1140,8 +1140,8 @@ void launch_mixed_chunked(lpm_ctx*, const PackedSources& src,
               nullptr};
   hipLaunchKernelGGL(eps2 > 0 ? bve_vel_mfma16_chunk_kernel<true>
                               : bve_vel_mfma16_chunk_kernel<false>,
-                     dim3(static_cast<unsigned>(a0.nblocks + a1.nblocks) *
-                          (split ? C : 1)),
+                     launch_grid((static_cast<int64_t>(a0.nblocks) +
+                                  a1.nblocks) * (split ? C : 1), 256),
                      dim3(256), 0, s, m, src.count, a0, a1,
                      static_cast<float>(2.0 * eps2), C);
   LPM_HIP_CHECK(hipGetLastError());
@@ -1290,7 +1290,7 @@ void launch_bve_stream_fn(lpm_ctx* ctx, const PackedSources& src,
   const int64_t nt = t0.n + t1.n;
   if (nt == 0) return;
   SegArgs a0 = to_args(t0, 64), a1 = to_args(t1, 64);
-  const int blocks = a0.nblocks + a1.nblocks;
+  const int64_t blocks = static_cast<int64_t>(a0.nblocks) + a1.nblocks;
   const int C = log_chunks(nt, src.capacity);
   // one chunk, or no workspace (a caller's capture, no memory): whole blocks
   double* part =
@@ -1303,8 +1303,8 @@ void launch_bve_stream_fn(lpm_ctx* ctx, const PackedSources& src,
   }
   TimedLaunch tl(ctx, KID_BVE_PSI, s, count_pairs(segs, nseg, src.capacity));
   hipLaunchKernelGGL(bve_psi_kernel,
-                     dim3(static_cast<unsigned>(blocks) * (part ? C : 1)),
-                     dim3(256), 0, s, static_cast<const double4*>(src.data),
+                     launch_grid(blocks * (part ? C : 1), 256), dim3(256), 0, s,
+                     static_cast<const double4*>(src.data),
                      ctx->log_table.as<double2>(), src.count, a0, a1, C);
   LPM_HIP_CHECK(hipGetLastError());
   if (part) {

@@ -113,8 +113,8 @@ __global__ __launch_bounds__(256) void ic2d_f64_kernel(
   __shared__ double2 ltab[kLogTable];
   __shared__ double red[4][4][64];
   const bool split = s0.part != nullptr;
-  const int b = split ? static_cast<int>(blockIdx.x) / C : blockIdx.x;
-  const int c0 = split ? static_cast<int>(blockIdx.x) % C : 0;
+  const int b = split ? flat_block() / C : flat_block();
+  const int c0 = split ? flat_block() % C : 0;
   const bool first = b < s0.nblocks;
   const SegArgs& sg = pick(s0, s1, first);
   const int blk = first ? b : b - s0.nblocks;
@@ -198,8 +198,8 @@ __global__ __launch_bounds__(256, 4) void ic2d_mixed_kernel(
   __shared__ uint4 la[2 * kPackTile];
   __shared__ float4 lt[kPackTile];
   const bool split = s0.part != nullptr;
-  const int b = split ? static_cast<int>(blockIdx.x) / C : blockIdx.x;
-  const int c0 = split ? static_cast<int>(blockIdx.x) % C : 0;
+  const int b = split ? flat_block() / C : flat_block();
+  const int c0 = split ? flat_block() % C : 0;
   const bool first = b < s0.nblocks;
   const SegArgs& sg = pick(s0, s1, first);
   const int blk = first ? b : b - s0.nblocks;
@@ -394,7 +394,7 @@ void launch_ic2d(lpm_ctx* ctx, const PackedSources& src, TargetSeg* segs,
     return a;
   };
   SegArgs a0 = to_args(t0), a1 = to_args(t1);
-  const int blocks = a0.nblocks + a1.nblocks;
+  const int64_t blocks = static_cast<int64_t>(a0.nblocks) + a1.nblocks;
   const int ks = ic2d_chunks(precision, t0.n + t1.n, src.capacity);
   // no workspace (a caller's capture, no memory): whole blocks, chunk by chunk
   double* part =
@@ -406,7 +406,7 @@ void launch_ic2d(lpm_ctx* ctx, const PackedSources& src, TargetSeg* segs,
   }
   const double pairs = static_cast<double>(t0.n + t1.n) * src.capacity;
   TimedLaunch tl(ctx, KID_IC2D, s, pairs);
-  const dim3 grid(static_cast<unsigned>(blocks) * (part ? ks : 1));
+  const dim3 grid = launch_grid(blocks * (part ? ks : 1), 256);
   if (precision == LPM_MIXED) {
     LPM_ARG_CHECK(src.mf_a && src.mf_g, "matrix-core layout not packed");
     Mfma16Src m{src.mf_y, src.mf_s,  src.mf_a, src.mf_t32,

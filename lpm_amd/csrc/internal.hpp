@@ -14,6 +14,7 @@
 #include <string>
 #include <vector>
 
+#include "launch_grid.hpp"
 #include "lpm_mi355x.h"
 
 namespace lpm_amd {
@@ -272,6 +273,18 @@ int default_variant(int family);
 std::string tune_key(const lpm_ctx* ctx, int family, int64_t n_targets);
 int pick_variant(lpm_ctx* ctx, int family, int64_t n_targets);
 hipStream_t as_stream(void* s);
+
+// grid_xy as a launch argument.
+inline dim3 launch_grid(int64_t blocks, int threads) {
+  const GridXY g = grid_xy(blocks, threads);
+  return dim3(g.x, g.y);
+}
+#ifdef __HIP__
+// Block index in such a launch.
+__device__ __forceinline__ int flat_block() {
+  return static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+}
+#endif
 
 // Event bracket for a timed launch (no-op when timing is off).
 struct TimedLaunch {

@@ -838,8 +838,8 @@ __global__ __launch_bounds__(64 * kSweWaves, 4) void swe_wave_kernel(
     const int32_t* __restrict__ count, SweSeg s0, SweSeg s1, SweParams P,
     int C) {
   __shared__ double red[kSweWaves / 2][kSweRows][64];
-  const int b = SPLIT ? static_cast<int>(blockIdx.x) / C : blockIdx.x;
-  const int k = SPLIT ? static_cast<int>(blockIdx.x) % C : 0;
+  const int b = SPLIT ? flat_block() / C : flat_block();
+  const int k = SPLIT ? flat_block() % C : 0;
   const bool first = b < s0.nblocks;
   const SweSeg& sg = first ? s0 : s1;
   const int blk = first ? b : b - s0.nblocks;
@@ -1587,8 +1587,8 @@ __global__ __launch_bounds__(BLOCK, MINW) void swe_mf_far_kernel(
     const SweSrc* __restrict__, const double4* __restrict__,
     const int32_t* __restrict__ count, SweSeg s0, SweSeg s1, SweParams P) {
   __shared__ uint4 buf[2][kSweMfRec];
-  const int b = static_cast<int>(blockIdx.x) / P.rows;
-  const int k0 = static_cast<int>(blockIdx.x) % P.rows;
+  const int b = flat_block() / P.rows;
+  const int k0 = flat_block() % P.rows;
   const bool first = b < s0.nblocks;
   const SweSeg& sg = first ? s0 : s1;
   const int blk = first ? b : b - s0.nblocks;
@@ -1605,9 +1605,10 @@ __global__ __launch_bounds__(256, MINW) void swe_mf_near_kernel(
     const int32_t* __restrict__ count, SweSeg s0, SweSeg s1, SweParams P) {
   __shared__ SweSrc stage[4 * kSweMfSub];
   __shared__ double red[2][kSweRows][64];
-  const bool first = static_cast<int>(blockIdx.x) < s0.nblocks;
+  const int b = flat_block();
+  const bool first = b < s0.nblocks;
   const SweSeg& sg = first ? s0 : s1;
-  const int blk = first ? blockIdx.x : blockIdx.x - s0.nblocks;
+  const int blk = first ? b : b - s0.nblocks;
   swe_mf_near_block<SHARE>(src, P.mf, *count, sg, blk, P.rows, P,
                            stage + (threadIdx.x & ~63), red);
 }
@@ -1746,7 +1747,8 @@ __global__ __launch_bounds__(64 * kSweWaves, 4) void swe_ens_wave_kernel(
     const double* __restrict__ src, const double4* __restrict__ sub,
     SweEnsArgs A, double* part) {
   __shared__ double red[kSweWaves / 2][kSweRows][64];
-  const int4 w = A.items[blockIdx.x];
+  if (flat_block() >= A.n_items) return;
+  const int4 w = A.items[flat_block()];
   const EnsMember M = A.mem[w.x];
   SweSeg sg = swe_ens_segment(A, M, w.y);
   if (SPLIT) swe_ens_parts(sg, M, w.y, part);
@@ -1756,7 +1758,8 @@ __global__ __launch_bounds__(64 * kSweWaves, 4) void swe_ens_wave_kernel(
 
 __global__ __launch_bounds__(64) void swe_ens_wave_reduce_kernel(SweEnsArgs A,
                                                                  double* part) {
-  const int4 w = A.items[blockIdx.x];
+  if (flat_block() >= A.n_items) return;
+  const int4 w = A.items[flat_block()];
   const EnsMember M = A.mem[w.x];
   SweSeg sg = swe_ens_segment(A, M, w.y);
   swe_ens_parts(sg, M, w.y, part);
@@ -1817,7 +1820,8 @@ template <int BLOCK, int MINW>
 __global__ __launch_bounds__(BLOCK, MINW) void swe_ens_mf_far_kernel(
     SweEnsArgs A, double* part) {
   __shared__ uint4 buf[2][kSweMfRec];
-  const int4 w = A.items[blockIdx.x];
+  if (flat_block() >= A.n_items) return;
+  const int4 w = A.items[flat_block()];
   const EnsMember M = A.mem[w.x];
   SweSeg sg = swe_ens_segment(A, M, w.y);
   swe_ens_far(sg, M, w.y, A, part);
@@ -1834,12 +1838,13 @@ __global__ __launch_bounds__(256, MINW) void swe_ens_mf_near_kernel(
     const SweSrc* __restrict__ src, SweEnsArgs A, double* part) {
   __shared__ SweSrc stage[4 * kSweMfSub];
   __shared__ double red[2][kSweRows][64];
-  const int4 w = A.items[blockIdx.x / 4];
+  if (flat_block() / 4 >= A.n_items) return;
+  const int4 w = A.items[flat_block() / 4];
   const EnsMember M = A.mem[w.x];
   SweSeg sg = swe_ens_segment(A, M, w.y);
   swe_ens_far(sg, M, w.y, A, part);
   swe_mf_near_block<SHARE>(src + M.P, A.P.mf.from(M.P / kSweTile), M.cnt, sg,
-                           4 * w.z + static_cast<int>(blockIdx.x % 4),
+                           4 * w.z + flat_block() % 4,
                            A.P.rows == 1 ? 1 : M.C, A.P,
                            stage + (threadIdx.x & ~63), red);
 }
@@ -2027,7 +2032,7 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
   constexpr int kBlock = 256;
   const int per = v.wave ? 64 : kBlock;
   SweSeg a0 = to_seg(t0, per), a1 = to_seg(t1, per);
-  const int grid = a0.nblocks + a1.nblocks;
+  const int64_t grid = static_cast<int64_t>(a0.nblocks) + a1.nblocks;
   const int do_pse = pse_eps > 0 ? 1 : 0;
   const double inv_e2 = do_pse ? 1.0 / (pse_eps * pse_eps) : 0.0;
   const double cut2 = do_pse ? kPseCut * pse_eps * pse_eps : 0.0;
@@ -2045,7 +2050,7 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
     a1.part = part + (part ? kSweRows * static_cast<int64_t>(C) * a0.n : 0);
     TimedLaunch tl(ctx, KID_SWE_F64, s, pairs);
     hipLaunchKernelGGL(part ? swe_wave_kernel<true> : swe_wave_kernel<false>,
-                       dim3(static_cast<unsigned>(grid) * (part ? C : 1)),
+                       launch_grid(grid * (part ? C : 1), 64 * kSweWaves),
                        dim3(64 * kSweWaves), 0, s,
                        static_cast<const double*>(src.data), src.bounds,
                        src.count, a0, a1, P, C);
@@ -2074,13 +2079,16 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
     a0.part = part ? part : swe_far_rows(ctx, nt);
     a1.part = a0.part + kSweMfRows * static_cast<int64_t>(P.rows) * a0.n;
     TimedLaunch tl(ctx, KID_SWE_MIXED, s, pairs);
-    hipLaunchKernelGGL(v.far, dim3(static_cast<unsigned>(grid) * P.rows),
+    hipLaunchKernelGGL(v.far, launch_grid(grid * P.rows, kBlock),
                        dim3(kBlock), 0, s, static_cast<const SweSrc*>(src.data),
                        src.bounds, src.count, a0, a1, P);
     LPM_HIP_CHECK(hipGetLastError());
     a0.nblocks = static_cast<int>((a0.n + 63) / 64);
     a1.nblocks = static_cast<int>((a1.n + 63) / 64);
-    hipLaunchKernelGGL(v.near, dim3(a0.nblocks + a1.nblocks), dim3(256), 0, s,
+    hipLaunchKernelGGL(v.near,
+                       launch_grid(static_cast<int64_t>(a0.nblocks) + a1.nblocks,
+                                   256),
+                       dim3(256), 0, s,
                        static_cast<const SweSrc*>(src.data), src.bounds,
                        src.count, a0, a1, P);
     LPM_HIP_CHECK(hipGetLastError());
@@ -2088,7 +2096,7 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
   }
   TimedLaunch tl(ctx, precision == LPM_FP64 ? KID_SWE_F64 : KID_SWE_MIXED, s,
                  pairs);
-  hipLaunchKernelGGL(v.fn, dim3(grid), dim3(kBlock), 0, s,
+  hipLaunchKernelGGL(v.fn, dim3(static_cast<unsigned>(grid)), dim3(kBlock), 0, s,
                      static_cast<const SweSrc*>(src.data), src.bounds,
                      src.count, a0, a1, P);
   LPM_HIP_CHECK(hipGetLastError());
@@ -2182,16 +2190,20 @@ void swe_ensemble_sums(lpm_ctx* ctx, const EnsembleDesc& d,
     double* part =
         chunk_workspace(ctx, sizeof(double) * kSweRows * L.parts, s);
     SweEnsArgs B = A;
-    if (part) B.items = L.chunk_items;
+    if (part) {
+      B.items = L.chunk_items;
+      B.n_items = L.n_chunk_items;
+    }
     TimedLaunch tl(ctx, KID_SWE_F64, s, L.pairs);
     hipLaunchKernelGGL(
         part ? swe_ens_wave_kernel<true> : swe_ens_wave_kernel<false>,
-        dim3(static_cast<unsigned>(part ? L.n_chunk_items : L.n_items)),
-        dim3(64 * kSweWaves), 0, s, reinterpret_cast<const double*>(src),
+        launch_grid(B.n_items, 64 * kSweWaves), dim3(64 * kSweWaves), 0, s,
+        reinterpret_cast<const double*>(src),
         static_cast<const double4*>(bounds), B, part);
     LPM_HIP_CHECK(hipGetLastError());
     if (part) {
-      swe_ens_wave_reduce_kernel<<<L.n_items, 64, 0, s>>>(A, part);
+      swe_ens_wave_reduce_kernel<<<launch_grid(L.n_items, 64), 64, 0, s>>>(A,
+                                                                        part);
       LPM_HIP_CHECK(hipGetLastError());
     }
     return;
@@ -2205,14 +2217,18 @@ void swe_ensemble_sums(lpm_ctx* ctx, const EnsembleDesc& d,
         chunk_workspace(ctx, sizeof(double) * kSweMfRows * L.parts, s);
     A.P.rows = part ? 0 : 1;  // 0: each member's chunks
     SweEnsArgs B = A;
-    if (part) B.items = L.chunk_items;
-    else part = swe_far_rows(ctx, d.n_verts + d.n_faces);
+    if (part) {
+      B.items = L.chunk_items;
+      B.n_items = L.n_chunk_items;
+    } else {
+      part = swe_far_rows(ctx, d.n_verts + d.n_faces);
+    }
     TimedLaunch tl(ctx, KID_SWE_MIXED, s, L.pairs);
-    hipLaunchKernelGGL(v.ens_far,
-                       dim3(A.P.rows == 1 ? L.n_items : L.n_chunk_items),
-                       dim3(kBlock), 0, s, B, part);
+    hipLaunchKernelGGL(v.ens_far, launch_grid(B.n_items, kBlock), dim3(kBlock),
+                       0, s, B, part);
     LPM_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(v.ens_near, dim3(4 * L.n_items), dim3(256), 0, s,
+    hipLaunchKernelGGL(v.ens_near,
+                       launch_grid(int64_t{4} * L.n_items, 256), dim3(256), 0, s,
                        static_cast<const SweSrc*>(src), A, part);
     LPM_HIP_CHECK(hipGetLastError());
     return;
