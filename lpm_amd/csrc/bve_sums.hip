@@ -749,7 +749,8 @@ const char* variant_name(int family, int v) {
 int default_variant(int family) {
   if (family == KID_BVE_ENS_F64 || family == KID_BVE_ENS_MIXED)
     return ens_default_variant(family);
-  if (family == KID_SWE_F64 || family == KID_SWE_MIXED) return 0;
+  if (family == KID_SWE_F64 || family == KID_SWE_MIXED)
+    return swe_default_variant(family);
   return family == KID_BVE_VEL_F64 ? kDefaultF64 : kDefaultMixed;
 }
 

@@ -578,6 +578,7 @@ void ensemble_velocity(lpm_ctx* ctx, const EnsembleDesc& d,
 // Kernel variants of KID_SWE_F64 / KID_SWE_MIXED (the default is 0).
 int swe_variant_count(int family);
 const char* swe_variant_name(int family, int v);
+int swe_default_variant(int family);
 struct SwePacked {
   const void* data = nullptr;       // 64 B per source
   const double4* bounds = nullptr;  // per 256-source tile: centre, radius^2

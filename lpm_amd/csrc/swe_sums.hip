@@ -1871,11 +1871,20 @@ struct SweVariant {
   }
 };
 constexpr int kSweBlock = 256;
+// The numbers are kept: programs and tuning tables hold them.
 const SweVariant kSweF64Variants[] = {
-    {nullptr, nullptr, "wave8_scalar", nullptr, nullptr, nullptr, nullptr, true},
     {swe_f64_kernel<kSweBlock, 4, 3>, swe_ens_f64_kernel<kSweBlock, 4, 3>,
      "share4_occ3"},
+    {swe_f64_kernel<kSweBlock, 4, 4>, swe_ens_f64_kernel<kSweBlock, 4, 4>,
+     "share4_occ4"},
+    {swe_f64_kernel<kSweBlock, 2, 4>, swe_ens_f64_kernel<kSweBlock, 2, 4>,
+     "share2_occ4"},
+    {swe_f64_kernel<kSweBlock, 2, 3>, swe_ens_f64_kernel<kSweBlock, 2, 3>,
+     "share2_occ3"},
+    // 4: the default
+    {nullptr, nullptr, "wave8_scalar", nullptr, nullptr, nullptr, nullptr, true},
 };
+constexpr int kDefaultSweF64 = 4;
 const SweVariant kSweMixedVariants[] = {
     // two passes: far tiles and sub-tiles on the matrix cores, then near
     // sub-tiles and PSE terms in FP64 and the outputs
@@ -1954,6 +1963,10 @@ const char* swe_variant_name(int family, int v) {
   if (v < 0 || v >= swe_variant_count(family)) return nullptr;
   return family == KID_SWE_F64 ? kSweF64Variants[v].name
                                : kSweMixedVariants[v].name;
+}
+
+int swe_default_variant(int family) {
+  return family == KID_SWE_F64 ? kDefaultSweF64 : 0;
 }
 
 void swe_feature_workspace(lpm_ctx* ctx, int64_t n_src, int64_t n_targets,

@@ -186,3 +186,25 @@ def test_mixed_stepper_without_renormalize_warns():
         warnings.simplefilter("error")
         Incompressible2DRK2(0.01, None, precision="mixed", renormalize=True)
         Incompressible2DRK2(0.01, None)
+
+
+def test_variant_numbers_are_kept():
+    """Programs and saved tuning tables hold kernel variants by number: new
+    ones are appended."""
+    L = _abi.lib()
+
+    def names(kid):
+        return [L.lpm_variant_name(kid, v).decode()
+                for v in range(L.lpm_variant_count(kid))]
+    first = {
+        _abi.LPM_KERNEL_SWE_F64: ["share4_occ3", "share4_occ4", "share2_occ4",
+                                  "share2_occ3"],
+        _abi.LPM_KERNEL_SWE_MIXED: ["mfma_f2n3", "mfma_f2n4", "occ4", "occ3",
+                                    "occ2"],
+    }
+    for kid, known in first.items():
+        assert names(kid)[:len(known)] == known
+    assert names(_abi.LPM_KERNEL_BVE_VEL_F64)[25] == \
+        "block256_tpl4_nr1_quad_fused_sy_u2_tile512_split32"
+    assert names(_abi.LPM_KERNEL_BVE_VEL_MIXED)[18] == \
+        "mfma16_occ5_qrcp_block256_near3"
