@@ -122,10 +122,11 @@ __device__ __forceinline__ double log_part(double a, const double2* tab,
 }
 
 // Screen of log_part's arguments: the largest log_screen(a) of a run is below
-// kLogScreen when every a was positive, finite and above 2^-1022.
-constexpr uint32_t kLogScreen = 0x7fefffffu;
+// kLogScreen when every a was positive, finite and at least 2^-1022 (subnormal
+// ones have high words below 0x00100000 and wrap, as zero and negative ones).
+constexpr uint32_t kLogScreen = 0x7fe00000u;
 __device__ __forceinline__ uint32_t log_screen(double a) {
-  return static_cast<uint32_t>(__double2hiint(a)) - 1u;
+  return static_cast<uint32_t>(__double2hiint(a)) - 0x00100000u;
 }
 
 // One source: S += s / (1 - x.y [+ eps^2]) * y.
