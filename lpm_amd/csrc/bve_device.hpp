@@ -502,6 +502,8 @@ constexpr int kQuadDoubles = 24;
 constexpr int kWaveTile = 16;  // quads per partial sum
 template <bool MESH>
 constexpr int kWaveRedo = MESH ? 0x3DB00000 : 0x3EB00000;  // 2^-36, 2^-20
+// Largest eps^2 with which four distances share a reciprocal.
+constexpr double kMaxShared = 0x1p250;
 
 // Quads [*q0, *q1) of wave w of chunk `chunk` of C.
 __device__ __forceinline__ void wave_range(int nq, int chunk, int C, int w,
@@ -659,6 +661,10 @@ __device__ __forceinline__ void wave_f64_block(
   const int nq = (nsrc + 3) / 4;
   const int64_t mine = slot0 + threadIdx.x;  // slot this thread reduces
   const bool owner = threadIdx.x < 64 * TPL && mine < n_live;
+  // smoothing so wide that a product of four distances would overflow: every
+  // tile pair by pair
+  const int redo =
+      EPS && eps2 > kMaxShared ? 0x7ff00000 : kWaveRedo<MESH>;
   double tot[3] = {0.0, 0.0, 0.0};
 #pragma unroll 1
   for (int chunk = c0; chunk < c1; ++chunk) {
@@ -684,12 +690,12 @@ __device__ __forceinline__ void wave_f64_block(
                                                low);
 #pragma unroll
       for (int k = 0; k < TPL; ++k)
-        if (__ballot(low[k] < kWaveRedo<MESH>)) {
+        if (__ballot(low[k] < redo)) {
           double R[3];
           wave_f64_redo(quads, q, e, x[k], self[k], eps2, R);
 #pragma unroll
           for (int a = 0; a < 3; ++a)
-            T[k][a] = low[k] < kWaveRedo<MESH> ? R[a] : T[k][a];
+            T[k][a] = low[k] < redo ? R[a] : T[k][a];
         }
 #pragma unroll
       for (int k = 0; k < TPL; ++k)

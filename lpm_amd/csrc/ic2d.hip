@@ -124,6 +124,8 @@ __global__ __launch_bounds__(256) void ic2d_f64_kernel(
   if (slot0 >= n_live) return;
   load_log_table(table, ltab);
   const double one_e = 1.0 + eps2;
+  // smoothing too wide for a shared reciprocal: every tile pair by pair
+  const uint32_t screen = eps2 > kMaxShared ? 0u : kLogScreen;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t c = slot0 + lane;
@@ -150,10 +152,10 @@ __global__ __launch_bounds__(256) void ic2d_f64_kernel(
       else
         ic2d_quads<false>(rec, q, e, x, one_e, self, ltab, T, top);
       double V[4] = {T.S[0], T.S[1], T.S[2], __builtin_fma(T.K, kLn2, T.R)};
-      if (__ballot(top >= kLogScreen)) {
+      if (__ballot(top >= screen)) {
         double D[3], psi;
         ic2d_redo(rec, q, e, x, one_e, self, D, psi);
-        if (top >= kLogScreen) {
+        if (top >= screen) {
           V[0] = D[0];
           V[1] = D[1];
           V[2] = D[2];
