@@ -405,7 +405,7 @@ bool issue_chunk_step(lpm_ctx* ctx, const lpm_bve_fields& f, double dt,
   PackArgs K{};
   PackedSources quad;
   if (layouts == kLayoutQuad) {
-    K = PackArgs{pack_workspace(ctx, layouts, f.n_faces, precision).quad,
+    K = PackArgs{pack_workspace(ctx, f.n_faces, precision).quad,
                  f.face_area, map.rank, map.d_count};
     quad.quad = K.quad;
     quad.count = map.d_count;
@@ -742,8 +742,7 @@ int lpm_bve_rk4_step(lpm_ctx* ctx, const lpm_bve_fields* f, double dt,
       rank_workspace(ctx, f->face_mask, f->n_faces);
       const int64_t nt = f->n_verts + f->n_faces;
       const int variant = bve_velocity_variant(ctx, precision, nt);
-      pack_workspace(ctx, bve_variant_layouts(precision, variant), f->n_faces,
-                     precision);
+      pack_workspace(ctx, f->n_faces, precision);
       if (precision == LPM_MIXED)
         target_order(ctx, vert_crd(*f), f->n_verts, nullptr, 1, s);
       const size_t part = bve_split_bytes(precision, variant, nt, f->n_faces);

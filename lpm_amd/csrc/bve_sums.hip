@@ -951,8 +951,7 @@ PackedSources pack_sources_into(const PackWs& ws, unsigned layouts, CrdIn sx,
   return ps;
 }
 
-PackWs pack_workspace(lpm_ctx* ctx, unsigned layouts, int64_t n,
-                      int precision) {
+PackWs pack_workspace(lpm_ctx* ctx, int64_t n, int precision) {
   const int64_t cap = std::max<int64_t>(n, 1);
   const int64_t ntile = (cap + kPackTile - 1) / kPackTile;
   const int64_t tcap = ntile * kPackTile;
@@ -961,40 +960,31 @@ PackWs pack_workspace(lpm_ctx* ctx, unsigned layouts, int64_t n,
     p = static_cast<std::remove_reference_t<decltype(p)>>(
         b.ensure(sizeof(*p) * count));
   };
-  if (layouts & kLayoutQuad)
-    buf(ctx->quad, ws.quad, (cap + 3) / 4 * kQuadDoubles);
-  if (layouts & kLayoutRec) buf(ctx->quad, ws.rec, (cap + 3) / 4 * 32);
-  if (layouts != kLayoutQuad && layouts != kLayoutRec &&
-      !(layouts & kLayoutMfma16))
-    buf(ctx->packed64, ws.p64, (cap + 3) / 4 * 4);
-  if (precision == LPM_FP64 && (layouts & kLayoutSy))
+  buf(ctx->packed64, ws.p64, (cap + 3) / 4 * 4);
+  if (precision == LPM_FP64) {
+    buf(ctx->quad, ws.rec, (cap + 3) / 4 * 32);
+    ws.quad = ws.rec;
     buf(ctx->packed64sy, ws.psy, cap);
-  if (layouts & kLayoutVec32) {
-    buf(ctx->packed32, ws.p32, cap);
-    buf(ctx->centers, ws.centers, ntile);
+    return ws;
   }
-  if (layouts & (kLayoutMfma | kLayoutMfma16)) {
-    buf(ctx->mf_y, ws.mf_y, tcap);
-    buf(ctx->mf_s, ws.mf_s, tcap);
-    buf(ctx->mf_c, ws.mf_c, ntile);
-  }
-  if (layouts & kLayoutMfma) {
-    buf(ctx->mf_q, ws.mf_q, tcap);
-    buf(ctx->mf_t, ws.mf_t, 4 * tcap);
-  }
-  if (layouts & kLayoutMfma16) {
-    buf(ctx->mf_a, ws.mf_a, 2 * tcap);
-    buf(ctx->mf_t32, ws.mf_t32, 4 * tcap);
-    buf(ctx->mf_is, ws.mf_is, ntile);
-  }
-  if (layouts & kLayoutLog) buf(ctx->mf_g, ws.mf_g, ntile);
+  buf(ctx->packed32, ws.p32, cap);
+  buf(ctx->centers, ws.centers, ntile);
+  buf(ctx->mf_y, ws.mf_y, tcap);
+  buf(ctx->mf_s, ws.mf_s, tcap);
+  buf(ctx->mf_c, ws.mf_c, ntile);
+  buf(ctx->mf_q, ws.mf_q, tcap);
+  buf(ctx->mf_t, ws.mf_t, 4 * tcap);
+  buf(ctx->mf_a, ws.mf_a, 2 * tcap);
+  buf(ctx->mf_t32, ws.mf_t32, 4 * tcap);
+  buf(ctx->mf_is, ws.mf_is, ntile);
+  buf(ctx->mf_g, ws.mf_g, ntile);
   return ws;
 }
 
 PackedSources pack_sources(lpm_ctx* ctx, unsigned layouts, CrdIn sx,
                            const double* zeta, const double* area,
                            const RankMap& map, int precision, hipStream_t s) {
-  return pack_sources_into(pack_workspace(ctx, layouts, map.n, precision),
+  return pack_sources_into(pack_workspace(ctx, map.n, precision),
                            layouts, sx, zeta, area, map, precision, s);
 }
 

@@ -643,7 +643,7 @@ int lpm_ic2d_rk2_step(lpm_ctx* ctx, const lpm_ic2d_fields* f, double dt,
         ctx, (flags & LPM_RK4_USE_GRAPH) != 0, s,
         [&]() {
           rank_workspace(ctx, f->face_mask, f->n_faces);
-          pack_workspace(ctx, ic2d_layouts(precision), f->n_faces, precision);
+          pack_workspace(ctx, f->n_faces, precision);
           // the split workspace of the two evaluations, before any capture
           const int ks =
               ic2d_chunks(precision, f->n_verts + f->n_faces, f->n_faces);

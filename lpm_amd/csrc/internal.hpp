@@ -353,8 +353,10 @@ struct PackWs {
   double* mf_is = nullptr;
   double4* mf_g = nullptr;
 };
-PackWs pack_workspace(lpm_ctx* ctx, unsigned layouts, int64_t n,
-                      int precision);
+// The context's own buffers of every layout of a precision (no launches), so
+// that a call of any kind or variant over n sources prepares the others: under a
+// caller's capture none of them allocates.
+PackWs pack_workspace(lpm_ctx* ctx, int64_t n, int precision);
 PackedSources pack_sources_into(const PackWs& ws, unsigned layouts, CrdIn sx,
                                 const double* zeta, const double* area,
                                 const RankMap& map, int precision,
