@@ -361,6 +361,17 @@ PackedSources pack_sources_into(const PackWs& ws, unsigned layouts, CrdIn sx,
                                 const double* zeta, const double* area,
                                 const RankMap& map, int precision,
                                 hipStream_t s);
+// Targets that fill the device by themselves (12 blocks of 256 per CU) over so
+// few sources that adding and storing chunk sums costs more than chunks gain:
+// one chunk.  1e6 free targets against 320, 1,280 and 5,120 sources, in
+// microseconds with chunks and without: FP64 velocity 134, 483, 1,708 and 117,
+// 419, 1,612; Incompressible2D 309, 1,199, 4,734 and 310, 1,111, 4,303; shallow
+// water 928, 3,598, 11,560 and 899, 2,961, 11,275; mixed velocity 154, 362,
+// 1,528 and 144, 350, 1,395.  At 20,480 sources chunks are as fast in FP64 and
+// 1.1 times as fast in mixed precision.
+inline bool one_chunk(int64_t n_targets, int64_t n_src) {
+  return n_targets >= (int64_t(3) << 18) && n_src <= 8192;
+}
 // Source chunks of the wave-split FP64 sums of a problem of n_targets
 // targets (both segments) and n_src stored sources: at least 16 (the chunk is
 // then fixed per XCD, block index mod 8, and its sources stay in that L2),
@@ -371,6 +382,7 @@ PackedSources pack_sources_into(const PackWs& ws, unsigned layouts, CrdIn sx,
 // sizes alone, so a member of an ensemble has the chunks (and bits) of its
 // one-problem call.
 inline int wave_chunks(int64_t n_targets, int64_t n_src) {
+  if (one_chunk(n_targets, n_src)) return 1;
   const int64_t blocks = (n_targets + 127) / 128;
   int64_t c = 16;
   while (c < 256 && blocks * c < 2048) c *= 2;
@@ -389,18 +401,21 @@ inline int log_chunks(int64_t n_targets, int64_t n_src) {
 // targets, tiles of 256 sources): 8 (the chunk is then fixed per XCD),
 // doubled until blocks times chunks reach 4,096 (three rounds of the resident
 // blocks), at most three quarters of the stored sources' tiles (a uniform
-// mesh's leaves), so that a chunk holds a tile or more.
+// mesh's leaves) or both of two, so that a chunk holds a tile or more.
 inline int mixed_chunks(int64_t n_targets, int64_t n_src) {
+  if (one_chunk(n_targets, n_src)) return 1;
   const int64_t blocks = (n_targets + 255) / 256;
-  const int64_t tiles = (n_src + 255) / 256 * 3 / 4;
+  const int64_t tiles = (n_src + 255) / 256;
   int64_t c = 8;
   while (c < 256 && blocks * c < 4096) c *= 2;
-  return static_cast<int>(std::max<int64_t>(1, std::min(c, tiles)));
+  c = std::min(c, tiles <= 2 ? tiles : tiles * 3 / 4);
+  return static_cast<int>(std::max<int64_t>(1, c));
 }
 // Source chunks of the wave-split FP64 shallow-water sums (eight waves of a
 // block share one): 8, doubled until the blocks of 64 targets times the
 // chunks reach 1,024 (four per CU) while every wave keeps 20 stored sources.
 inline int swe_chunks(int64_t n_targets, int64_t n_src) {
+  if (one_chunk(n_targets, n_src)) return 1;
   const int64_t blocks = (n_targets + 63) / 64;
   int64_t c = 8;
   while (c < 128 && blocks * c < 1024) c *= 2;
