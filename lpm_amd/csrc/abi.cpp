@@ -114,13 +114,17 @@ std::string tune_key(const lpm_ctx* ctx, int family, int64_t n_targets) {
   return ctx->arch + "/" + std::to_string(family) + "/" + std::to_string(b);
 }
 
-int pick_variant(lpm_ctx* ctx, int family, int64_t n_targets) {
+int pick_variant(lpm_ctx* ctx, int family, int64_t n_targets, int dflt) {
   if (ctx->forced[family] >= 0) return ctx->forced[family];
   auto it = ctx->tuned.find(tune_key(ctx, family, n_targets));
   if (it != ctx->tuned.end() && it->second >= 0 &&
       it->second < variant_count(family))
     return it->second;
-  return default_variant(family);
+  return dflt;
+}
+
+int pick_variant(lpm_ctx* ctx, int family, int64_t n_targets) {
+  return pick_variant(ctx, family, n_targets, default_variant(family));
 }
 
 TimedLaunch::TimedLaunch(lpm_ctx* c, int k, hipStream_t s, double p)

@@ -271,6 +271,8 @@ int variant_count(int family);
 const char* variant_name(int family, int v);
 int default_variant(int family);
 std::string tune_key(const lpm_ctx* ctx, int family, int64_t n_targets);
+// The forced or tuned variant, else dflt (default_variant).
+int pick_variant(lpm_ctx* ctx, int family, int64_t n_targets, int dflt);
 int pick_variant(lpm_ctx* ctx, int family, int64_t n_targets);
 hipStream_t as_stream(void* s);
 
@@ -618,7 +620,9 @@ void swe_sums_workspace(lpm_ctx* ctx, int64_t n_src, int64_t n_targets,
                         int precision, hipStream_t s);
 // Bounding spheres the sums read next to the packed sources.
 enum SweBounds : int { kSweNoBounds, kSweTileBounds, kSweRunBounds };
-SweBounds swe_bounds(lpm_ctx* ctx, int precision, int64_t n_targets);
+// n_src: the sources of a call with arbitrary targets, else -1.
+SweBounds swe_bounds(lpm_ctx* ctx, int precision, int64_t n_targets,
+                     int64_t n_src);
 // The packing's buffers, sized (no launches).
 void swe_pack_workspace(lpm_ctx* ctx, int64_t n_src);
 SwePacked swe_pack_sources(lpm_ctx* ctx, CrdIn sx, const double* zeta,

@@ -264,7 +264,7 @@ void sums_eval(lpm_ctx* ctx, const lpm_swe_fields& f, CrdIn vx, CrdIn fx,
                unsigned flags, hipStream_t s) {
   SwePacked ps = swe_pack_sources(
       ctx, fx, fzeta, fsigma, farea, f.face_surf, map,
-      swe_bounds(ctx, precision, f.n_verts + f.n_faces), s);
+      swe_bounds(ctx, precision, f.n_verts + f.n_faces, -1), s);
   SweTargets segs[2];
   segs[0].base.x = vx;
   segs[0].base.n = f.n_verts;
@@ -531,7 +531,7 @@ int lpm_swe_sphere_sums(lpm_ctx* ctx, const double* tgt_x, int64_t tgt_es,
     const RankMap map = build_rank(ctx, src_mask, n_src, s);
     SwePacked ps = swe_pack_sources(ctx, CrdIn{src_x, src_es, src_cs},
                                     src_zeta, src_sigma, src_area, src_surf,
-                                    map, swe_bounds(ctx, precision, n_tgt),
+                                    map, swe_bounds(ctx, precision, n_tgt, n_src),
                                     s);
     SweTargets t;
     if (collocated) {

@@ -1906,9 +1906,30 @@ constexpr int kNumSweF64 = sizeof(kSweF64Variants) / sizeof(kSweF64Variants[0]);
 constexpr int kNumSweMixed =
     sizeof(kSweMixedVariants) / sizeof(kSweMixedVariants[0]);
 
-const SweVariant& swe_variant(lpm_ctx* ctx, int precision, int64_t n_targets) {
+// Targets enough to fill the device with one wave for all sources of its
+// targets, over too few sources to divide among eight waves: share4_occ3 is
+// the faster FP64 form, and over a tile's half also faster than the mixed
+// passes.  For arbitrary points only (n_src, else -1): a mesh has no such
+// sizes, and a member of an ensemble keeps the bits of its problem alone.
+// 1e5 and 1e6 targets against 20 and 80 sources: 38, 46 and 84, 237 us, eight
+// waves 65, 77 and 452, 542, mixed 72, 93 and 362, 499; 5,000 targets 34 to 38
+// in FP64 either way.  1e6 against 320: 857, eight waves 926, mixed 844.
+bool swe_few_sources(int64_t n_targets, int64_t n_src, int precision) {
+  if (n_src < 0 || n_targets < 32768) return false;
+  return n_src <= 128 || (precision == LPM_FP64 &&
+                          one_chunk(n_targets, n_src) && n_src <= 512);
+}
+
+// Variant of a launch; n_src: its sources where the targets are arbitrary
+// points (else -1).
+const SweVariant& swe_variant(lpm_ctx* ctx, int precision, int64_t n_targets,
+                              int64_t n_src = -1) {
   const int family = precision == LPM_FP64 ? KID_SWE_F64 : KID_SWE_MIXED;
-  const int v = pick_variant(ctx, family, n_targets);
+  int v = pick_variant(ctx, family, n_targets, -1);
+  if (v < 0) {
+    if (swe_few_sources(n_targets, n_src, precision)) return kSweF64Variants[0];
+    v = swe_default_variant(family);
+  }
   if (precision == LPM_FP64) {
     LPM_ARG_CHECK(v >= 0 && v < kNumSweF64, "variant out of range");
     return kSweF64Variants[v];
@@ -1978,8 +1999,9 @@ void swe_feature_workspace(lpm_ctx* ctx, int64_t n_src, int64_t n_targets,
   ctx->swe_feat.ensure(kSweMfTileBytes * ntile);
 }
 
-SweBounds swe_bounds(lpm_ctx* ctx, int precision, int64_t n_targets) {
-  const SweVariant& v = swe_variant(ctx, precision, n_targets);
+SweBounds swe_bounds(lpm_ctx* ctx, int precision, int64_t n_targets,
+                     int64_t n_src) {
+  const SweVariant& v = swe_variant(ctx, precision, n_targets, n_src);
   return v.wave ? kSweRunBounds : v.mf() ? kSweNoBounds : kSweTileBounds;
 }
 
@@ -2041,7 +2063,8 @@ void launch_swe_sums(lpm_ctx* ctx, const SwePacked& src, SweTargets* segs,
   const SweTargets& t1 = nseg > 1 ? segs[1] : empty;
   const int64_t nt = t0.base.n + t1.base.n;
   if (nt == 0) return;
-  const SweVariant& v = swe_variant(ctx, precision, nt);
+  const SweVariant& v =
+      swe_variant(ctx, precision, nt, nseg == 1 ? src.capacity : -1);
   constexpr int kBlock = 256;
   const int per = v.wave ? 64 : kBlock;
   SweSeg a0 = to_seg(t0, per), a1 = to_seg(t1, per);

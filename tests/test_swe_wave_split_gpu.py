@@ -142,3 +142,27 @@ def test_without_a_workspace_the_bits_are_the_same(prec):
         del g
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("ns", [1, 5, 127, 128, 129])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_many_targets_over_few_sources(ctx, ora, ns, prec):
+    """From 32,768 arbitrary targets on, 128 sources or fewer are summed by one
+    wave for all of them, in FP64 also where mixed precision is asked for."""
+    m, x, area, zeta, sigma, surf = _inputs(ns, 4)
+    t = np.tile(m.vert_x, 13)[:, :32769]
+    src = [dev(a) for a in (x, zeta, sigma, area, surf(x))]
+    kw = dict(eps=0.05, pse_eps=0.3, precision=prec)
+    ref = ora.swe_sums(aos(t[:, :2562]), surf(t[:, :2562]), aos(x), zeta, sigma,
+                       area, surf(x), np.zeros(ns, np.uint8), eps=0.05,
+                       pse_eps=0.3)
+    for n in (32767, 32768, 32769):
+        got = ctx.swe_sums(dev(t[:, :n]), dev(surf(t[:, :n])), *src, **kw)
+        for g, r in zip(got, ref):
+            g = g.cpu().numpy()
+            # (the matrix-core passes' near tiles depend on a wave's targets)
+            few = prec == "fp64" or (n >= 32768 and ns <= 128)
+            if few:
+                assert np.array_equal(g[..., 2562:5124], g[..., :2562])
+            assert (np.linalg.norm(g[..., :2562].T - r) <=
+                    (TOL if few else 1e-6) * np.linalg.norm(r))
