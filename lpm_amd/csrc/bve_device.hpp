@@ -1256,16 +1256,12 @@ __global__ __launch_bounds__(kPackTile) void pack_mfma16_faces_kernel(
 // and a line that another XCD has just packed is 2,000 cycles away.  5,000 free
 // targets against 320 sources: 54 -> 37 us (49 with whole tiles staged in LDS,
 // 34 and 31 against 20 to 80); a level-6 step 7.00 -> 6.91 ms.
-// The statement without an instruction makes `use` wait for the load (it is not
-// volatile, which would count as a write to memory and turn the scalar loads
-// into vector loads).
-__device__ __forceinline__ void mfma16_touch(const float4* __restrict__ y,
-                                             const float* __restrict__ s,
-                                             int lane, float& use) {
+__device__ __forceinline__ float mfma16_touch(const float4* __restrict__ y,
+                                              const float* __restrict__ s,
+                                              int lane) {
   static_assert(kPackTile == 256, "32 lines of offsets, 8 of strengths");
-  const float* p = lane < 32 ? reinterpret_cast<const float*>(y) + 32 * lane
-                             : s + 32 * (min(lane, 39) - 32);
-  asm("" : "+v"(use) : "v"(*p));
+  return *(lane < 32 ? reinterpret_cast<const float*>(y) + 32 * lane
+                     : s + 32 * (min(lane, 39) - 32));
 }
 
 // Difference form d = y' - x' on the vector ALUs over the kPackTile sources of
@@ -1503,17 +1499,21 @@ __device__ __forceinline__ void mfma16_tiles(const Mfma16Src& src, int jbeg,
     const double inv = src.is[t];
     if (__ballot(mfma16_is_near<EPS>(e0 * e0 + e1 * e1 + ez * ez, inv, eps2x2))) {
       float T0 = 0.0f, T1 = 0.0f, T2 = 0.0f, T3 = 0.0f;
-      float xr0 = static_cast<float>(e0);
-      mfma16_touch(src.y + j0, src.s + j0, lane, xr0);
+      const float touch = mfma16_touch(src.y + j0, src.s + j0, lane);
       const auto near = [&](auto check) {
         mfma16_near<EPS, PSI, decltype(check)::value>(
-            src.y + j0, src.s + j0, xr0, static_cast<float>(e1),
-            static_cast<float>(ez), eps2x2, self - j0, T0, T1, T2, e2, &T3);
+            src.y + j0, src.s + j0, static_cast<float>(e0),
+            static_cast<float>(e1), static_cast<float>(ez), eps2x2, self - j0,
+            T0, T1, T2, e2, &T3);
       };
       if (__ballot(static_cast<unsigned>(self - j0) < unsigned{kPackTile}))
         near(std::true_type{});
       else
         near(std::false_type{});
+      // a use of the loaded value after the sums, without an instruction and
+      // not volatile (which would count as a write to memory and turn the
+      // scalar loads into vector loads)
+      asm("" : "+v"(T0) : "v"(touch));
       if (PSI) S3 += static_cast<double>(T3) * (0.5 * kLn2);
       S0 += static_cast<double>(T0);
       S1 += static_cast<double>(T1);
