@@ -565,7 +565,7 @@ __device__ __forceinline__ void wave_f64_quads(const double* __restrict__ quads,
 }
 
 // Quads [qa, qb) for one target, pair by pair with 1 - (x.y) + eps^2 in the
-// order of the pair formula and two Newton steps.
+// order of the pair formula, rounded as in f64_one, and two Newton steps.
 __device__ __forceinline__ void wave_f64_redo(const double* __restrict__ quads,
                                               int qa, int qb, const double* x,
                                               int self, double eps2,
@@ -575,7 +575,7 @@ __device__ __forceinline__ void wave_f64_redo(const double* __restrict__ quads,
   for (int j = 4 * qa; j < 4 * qb; ++j) {
     const double* y = quads + static_cast<int64_t>(j) * 6;
     const double t = __builtin_fma(
-        x[2], y[2], __builtin_fma(x[1], y[1], x[0] * y[0]));
+        x[2], y[2], __builtin_fma(x[0], y[0], x[1] * y[1]));
     const double r = rcp_nr<2>((1.0 - t) + eps2);
     const double w = j == self ? 0.0 : r;
 #pragma unroll
