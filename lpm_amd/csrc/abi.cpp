@@ -82,7 +82,6 @@ hipError_t DevBuf::release() {
   void* p = ptr;
   ptr = nullptr;
   bytes = 0;
-  g_workspace_epoch.fetch_add(1);
   if (!kept || !kept->recorded(born)) return hipFree(p);
   kept->ptrs.push_back(p);
   return hipSuccess;
@@ -92,7 +91,12 @@ DevBuf::~DevBuf() { (void)release(); }
 
 void* DevBuf::ensure(size_t nbytes) {
   if (nbytes <= bytes && ptr) return ptr;
-  LPM_HIP_CHECK(release());
+  if (ptr) {
+    // counted before the memory is gone, also if what follows fails; not in
+    // release(), as a context's end concerns no other context's graphs
+    g_workspace_epoch.fetch_add(1);
+    LPM_HIP_CHECK(release());
+  }
   const size_t want = std::max<size_t>(nbytes, 256);
   hipError_t e = hipMalloc(&ptr, want);
   if (e != hipSuccess) {

@@ -37,7 +37,7 @@ struct Error : std::runtime_error {
     if (!(cond)) throw ::lpm_amd::Error(LPM_ERR_ARG, (msg));      \
   } while (0)
 
-// Incremented whenever any workspace is allocated or given up; captured graphs
+// Incremented whenever any workspace is allocated or outgrown; captured graphs
 // record it and are re-captured when it changed, so that a replay never
 // touches freed workspace memory.
 extern std::atomic<uint64_t> g_workspace_epoch;
