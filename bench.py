@@ -125,7 +125,7 @@ def run_precision(ctx, mesh, precision, steps, warmup, dt, flags_extra,
 
 def ensemble_run(ctx, steps, warmup, dt=0.01, autotune=True):
     """64-member ensemble (icosahedral levels 3-6, RH 5-4 with random
-    omega, K and pattern rotation), one persistent launch per evaluation,
+    omega, K and pattern rotation), one launch per evaluation and its chunk sums,
     graph-captured RK4; mixed precision timed, FP64 for the error."""
     import numpy as np
     import torch
@@ -326,8 +326,8 @@ def swe_variant_sweep(ctx, e, prec, flags, reps=1):
 def swe_ensemble_run(ctx, steps=10, warmup=1, dt=0.005, level=6, members=16,
                      oracle_stride=64, tune=True):
     """Shallow water: 16 steady zonal (TC2) states on the icosahedral mesh of
-    level 6 with seeded 1e-4 height noise, one persistent launch per
-    evaluation, graph-captured RK4; mixed timed, FP64 for the error."""
+    level 6 with seeded 1e-4 height noise, one launch per evaluation and its
+    chunk sums, graph-captured RK4; mixed timed, FP64 for the error."""
     import numpy as np
     import torch
     from lpm_amd import _abi
@@ -995,7 +995,9 @@ def main(argv=None):
             # a source-split variant is two launches (partial sums, then
             # their reduction); avg_launch_ms times both
             "kernel": ("bve_vel_f64_split_kernel + bve_split_reduce_kernel"
-                       if "_split" in v64 else "bve_vel_f64_kernel"),
+                       if "_split" in v64 else
+                       "bve_wave_f64_kernel + bve_wave_reduce_kernel"
+                       if v64.startswith("wave") else "bve_vel_f64_kernel"),
             "variant": v64,
             "avg_launch_ms": round(avg_ms, 4),
             "flops_per_pair": F_BVE,

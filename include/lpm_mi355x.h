@@ -29,17 +29,20 @@
  *    this way: order such streams yourself.  Workspaces that such a call has
  *    recorded stay allocated until the context is destroyed, also when later
  *    calls outgrow them, so the caller's graph can be replayed that long.
- *  - Sums whose target blocks would leave the device underfilled split each
- *    block's sources into chunks and add the chunk partials in a second
- *    kernel (the stream function and Incompressible2D sums always when
- *    they have fewer target blocks than eight rounds of the blocks the
- *    device holds at once; BVE velocities in FP64 by default, and through the
- *    *_splitK variants).
- *    The partials live in a context workspace grown on demand; a call that
- *    cannot grow it (on a stream the caller is capturing, or out of device
- *    memory) runs unsplit (the FP64 default with the same chunks in one
- *    block, so with the same bits).  The chunk count follows from the problem
- *    size and the device, so results are reproducible on one device.
+ *  - The default sums divide the sources into chunks and add the chunk
+ *    partials in a second kernel.  The chunk count follows from the numbers
+ *    of targets and stored sources alone, so results are reproducible, and a
+ *    member of an ensemble has the bits of its problem alone.  The partials
+ *    live in a context workspace grown on demand to at most 1 GiB; a call
+ *    that needs more or cannot grow it (on a stream the caller is capturing,
+ *    or out of device memory) sums every chunk within a block, to the same
+ *    bits.  The *_splitK velocity variants run their unsplit twin without
+ *    their workspace.
+ *  - lpm_bve_velocity and lpm_bve_velocity_noalloc take points in any order;
+ *    the entry points on fields take the particles of a mesh in its order,
+ *    neighbours in memory near each other.  In FP64 both form 1 - x.y of
+ *    close pairs as the pair formula does, the former at every distance below
+ *    2^-20.
  */
 #ifndef LPM_MI355X_H
 #define LPM_MI355X_H
@@ -289,9 +292,9 @@ int lpm_bve_rk4_step(lpm_ctx* ctx, const lpm_bve_fields* f, double dt,
  * its velocity is the sum over its own undivided faces only.  The offset
  * arrays are host memory of n_members + 1 nondecreasing entries from 0 to
  * n_verts / n_faces; every member owns at least one face.
- * All members are evaluated by one persistent kernel that takes
- * (member, target block) work items from a queue, largest members first,
- * so members of very different sizes share one launch.  The work list is
+ * All members are evaluated by one launch over (member, target block, source
+ * chunk) work items, largest members first, so members of very different
+ * sizes share it, and one that adds the chunk sums.  The work list is
  * uploaded (synchronously) the first time an offset layout is seen and
  * cached in the context.
  * No reference counterpart: the reference evolves one BVESphere at a time
@@ -477,8 +480,9 @@ int lpm_swe_rk2_step(lpm_ctx* ctx, const lpm_swe_fields* f, double dt,
                      int precision, unsigned flags, void* stream);
 
 /* Ensembles of sphere SWE problems stored back to back, as
- * lpm_bve_ensemble (same offset rules): one persistent launch evaluates the
- * sums of every member.  No reference counterpart; each member's results
+ * lpm_bve_ensemble (same offset rules): one launch evaluates the sums of
+ * every member and one adds the chunk sums (two passes in mixed precision).
+ * No reference counterpart; each member's results
  * equal lpm_swe_init_sums / lpm_swe_rk4_step on that member alone, bit for
  * bit. */
 typedef struct lpm_swe_ensemble {
@@ -510,9 +514,12 @@ int lpm_swe_ensemble_rk2_step(lpm_ctx* ctx, const lpm_swe_ensemble* e,
  * context.  lpm_bve_init_velocity and lpm_bve_rk4_step run them (the step
  * sizes the workspace before any graph capture); lpm_bve_velocity and
  * lpm_bve_velocity_noalloc run the unsplit variant of the same shape.
- * wave4_scalar (the FP64 default) divides the sources among a block's waves
- * and, by a rule on the sizes, among blocks; every entry point runs it with
- * the same chunks and bits. */
+ * wave4_scalar and mfma16_chunked_near3 (the FP64 and mixed defaults) divide
+ * the sources by a rule on the sizes; every entry point runs them with the
+ * same chunks and bits.  The shallow-water defaults are wave8_scalar and
+ * mfma_f2n3; lpm_swe_sphere_sums runs share4_occ3 for 32,768 targets and more
+ * over 128 sources or fewer.  Variants keep their numbers; new ones are
+ * appended. */
 int lpm_variant_count(int kernel_id);
 const char* lpm_variant_name(int kernel_id, int variant);
 /* The variant used when nothing was tuned or forced. */

@@ -143,7 +143,7 @@ class BVERK4:
 
 class BVEEnsemble:
     """Independent BVE problems on the unit sphere stored back to back and
-    evaluated by one persistent launch per direct sum
+    evaluated by one launch per direct sum and one that adds its chunks
     (``lpm_bve_ensemble_*``).  Member m owns vertices
     ``vert_offsets[m]:vert_offsets[m+1]`` and faces
     ``face_offsets[m]:face_offsets[m+1]`` of the concatenated (3, n) / (n,)

@@ -1,6 +1,6 @@
-// BVE ensembles: every member's velocity from one persistent launch.  The
-// member layout and work plan come from ensemble.hip; a work item runs the
-// same block loop (bve_device.hpp) on the same target slots and source tiles
+// BVE ensembles: every member's velocity from one launch (and one that adds the
+// chunk sums).  The member layout and work plan come from ensemble.hip; a work
+// item runs the same block loop (bve_device.hpp) on the same target slots and source tiles
 // as a one-member launch, so results agree bit for bit with
 // lpm_bve_init_velocity on each member alone.
 #include <hip/hip_runtime.h>
@@ -313,6 +313,9 @@ struct EnsVariant {
   }
 };
 
+// Names are "persistent_" and the one-problem variant's, also of the shapes
+// whose blocks take one item (and chunk) each: wave4_scalar and
+// mfma16_chunked_near3, the defaults.
 #define LPM_ENS_F64(B, T, NR, PAIR)                  \
   {ens_f64_kernel<B, T, NR, PAIR>, nullptr, B, T,    \
    "persistent_block" #B "_tpl" #T "_nr" #NR "_pair" #PAIR, nullptr}
@@ -321,7 +324,7 @@ struct EnsVariant {
    "persistent_block" #B "_tpl" #T "_pair" #PAIR, nullptr}
 
 const EnsVariant kEnsF64[] = {
-    LPM_ENS_F64(256, 2, 2, true),  // 0: fixed default
+    LPM_ENS_F64(256, 2, 2, true),  // 0
     LPM_ENS_F64(256, 2, 1, true),  // 1
     LPM_ENS_F64(256, 1, 1, true),  // 2
     LPM_ENS_F64(256, 4, 1, true),  // 3
@@ -340,7 +343,7 @@ const EnsVariant kEnsF64[] = {
      true},
 };
 const EnsVariant kEnsMixed[] = {
-    LPM_ENS_MIXED(256, 2, false),  // 0: fixed default
+    LPM_ENS_MIXED(256, 2, false),  // 0
     LPM_ENS_MIXED(256, 1, true),   // 1
     LPM_ENS_MIXED(256, 1, false),  // 2
     LPM_ENS_MIXED(256, 2, true),   // 3

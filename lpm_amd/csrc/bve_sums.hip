@@ -719,9 +719,9 @@ constexpr int kNumMixed = sizeof(kMixedVariants) / sizeof(kMixedVariants[0]);
 // against 93 us for variant 1) to 1.6e11 (45 ms; variant 25 48.5, variant 1
 // 70).  The others keep their numbers: saved tuning tables hold them.
 constexpr int kDefaultF64 = 26;
-// The mixed default is the matrix-core kernel: 1.45 ms per level-6 evaluation
+// The mixed default is the matrix-core kernel: 1.71 ms per level-6 evaluation
 // against 5.67 for the vector form of variant 0, with a smaller error (tile
-// offsets from the centroid), and from level 3 up never slower.
+// offsets from the centroid); 23 against 36 us at level 1.
 constexpr int kDefaultMixed = 19;
 
 }  // namespace

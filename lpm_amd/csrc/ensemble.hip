@@ -7,10 +7,11 @@
 // the compacted ranks [R_m, R_m + cnt_m).  Each member's sources are packed
 // into their own region starting at P_m, a multiple of the 256-source
 // packing tile, so that every member's tiles are exactly those a
-// one-member call would build.  A persistent kernel takes (member, segment,
-// target block) work items from a queue through one atomic counter; items
-// are ordered by decreasing member face count, so the largest members start
-// first and small ones fill the tail.
+// one-member call would build.  A work item is (member, segment, target block)
+// or, of sums in chunks, one source chunk of it: a block each, or taken from a
+// queue through one atomic counter by the persistent kernels of the other
+// variants.  Items are ordered by decreasing member face count, so the largest
+// members start first and small ones fill the tail.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -483,8 +483,8 @@ double* split_workspace(lpm_ctx* ctx, size_t need, hipStream_t s);
 // shallow water of 1e7 targets would hold 12.8 GB.  At the bound, 2.8 million
 // targets in FP64 velocity and 839,000 in shallow water, the target blocks
 // alone fill the device many times.  Whole blocks against chunks: level 5
-// 1.3 to 3.9 times as long, level 6 1.08 to 1.6, level 7 (491,522 targets, 189
-// and 629 MB) 1.02 to 1.17; 1e6 and more targets 0.84 to 1.14.
+// 1.3 to 3.9 times as long, level 6 1.08 to 1.6, level 7 (600,742 slots, 231
+// and 769 MB) 1.02 to 1.17; 1e6 and more targets 0.84 to 1.14.
 constexpr size_t kChunkBytes = size_t(1) << 30;
 double* chunk_workspace(lpm_ctx* ctx, size_t need, hipStream_t s);
 // Uploads the table of the FP64 logarithm (context creation).

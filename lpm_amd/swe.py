@@ -178,7 +178,7 @@ class SWERK2(SWERK4):
 
 class SWEEnsemble(SWE):
     """Independent sphere SWE problems stored back to back (same field names
-    as SWE, concatenated), evaluated by one persistent launch per direct sum
+    as SWE, concatenated), evaluated by one launch per direct sum and one that adds its chunks
     (``lpm_swe_ensemble_*``).  Member m owns vertices
     ``vert_offsets[m]:vert_offsets[m+1]`` and faces
     ``face_offsets[m]:face_offsets[m+1]``.  No reference counterpart."""
