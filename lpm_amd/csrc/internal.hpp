@@ -425,16 +425,21 @@ inline int swe_chunks(int64_t n_targets, int64_t n_src) {
   return static_cast<int>(c);
 }
 // Source chunks of the shallow-water sums' matrix-core far pass (blocks of 256
-// targets, tiles of 256 sources): 1, doubled until blocks times chunks reach
-// 4,096 (eight rounds of the two resident blocks per CU), at most three
-// quarters of the stored sources' tiles.  The far sums of all chunks take
-// 144 C bytes a target, so at most 300 MB where C > 1.
+// targets, tiles of 256 sources): 8 (the chunk is then fixed per XCD), doubled
+// until blocks times chunks reach 2,048 (four rounds of the two resident blocks
+// per CU), at least two of three quarters of the stored sources' tiles a chunk
+// above eight of them; 1 from 4,096 blocks on.  Sums of level 5 in
+// microseconds for 2,048, 4,096: 546, 601; level 6 with 8, 4 chunks: 4,578,
+// 4,648; 30 problems of level 4 with at least 1, 2 tiles a chunk: 2,052, 1,770;
+// level 3 (five tiles) 117, 123.
 inline int swe_mf_chunks(int64_t n_targets, int64_t n_src) {
   const int64_t blocks = (n_targets + 255) / 256;
   const int64_t tiles = (n_src + 255) / 256 * 3 / 4;
-  int64_t c = 1;
-  while (c < 128 && blocks * c < 4096) c *= 2;
-  return static_cast<int>(std::max<int64_t>(1, std::min(c, tiles)));
+  if (blocks >= 4096) return 1;
+  int64_t c = 8;
+  while (c < 128 && blocks * c < 2048) c *= 2;
+  c = std::min(c, tiles <= 8 ? tiles : tiles / 2);
+  return static_cast<int>(std::max<int64_t>(1, c));
 }
 // Whether a velocity variant sums the sources in chunks by size.
 bool bve_variant_chunked(int precision, int variant);

@@ -1034,7 +1034,7 @@ __global__ __launch_bounds__(BLOCK, MINW) void swe_mixed_kernel(
 // Tile records (one 256-source tile each):
 //   cen        double4  (c, R^2)
 //   scen[4]    double4  sub-tile (c_s, r_s^2), r_s^2 = -1 without sources
-// and in one piece, which a block copies to LDS:
+// and in one piece:
 //   ya[256]    float4   (y - c, |y - c|^2 / 2); padding (8, 8, 8, 96)
 //   yas[256]   float4   the same relative to the source's sub-tile centroid
 //   fr[384]    uint4    set 1, [k-block 8][hi/lo][g 4][row 6] x 8 f16
@@ -1236,13 +1236,13 @@ __device__ __forceinline__ void add_qyq(double* G, const double* Y,
   }
 }
 
-// Far sums of k-blocks kb0 .. kb1 - 1 of one tile (its record rec in LDS; ya:
-// the record's offsets from the centroid c of the tile or sub-tile summed) for
-// the wave's four groups of 16 targets, carried into F1 / F2: lane (g, col)
+// Far sums of k-blocks kb0 .. kb1 - 1 of one tile (its record rec, whose operands
+// are fetched a k-block ahead; ya: the record's offsets from the centroid c of
+// the tile or sub-tile summed) for the wave's four groups of 16 targets, carried into F1 / F2: lane (g, col)
 // holds rows 4 g + v of target 16 G + col.  e is this lane's target minus c,
 // dist2 = |e|^2, R2 = the radius^2 around c.
 __device__ __forceinline__ void swe_mf_far_tile(
-    const uint4* rec, const float* ya, int kb0, int kb1, bool in, double e0,
+    const uint4* __restrict__ rec, const float* __restrict__ ya, int kb0, int kb1, bool in, double e0,
     double e1, double e2, double dist2, double R2, double eps2, int col, int g,
     double (*F1)[4], double (*F2)[4]) {
   constexpr int NG = 4;
@@ -1281,14 +1281,30 @@ __device__ __forceinline__ void swe_mf_far_tile(
   // lanes of unused rows repeat the last row: their results are not read
   const uint4* fr = rec + kSweMfFrAt + g * kSweMfR1 + min(col, kSweMfR1 - 1);
   const uint4* fr2 = rec + kSweMfFr2At + g * kSweMfR2 + min(col, kSweMfR2 - 1);
+  struct Operands {
+    float a0, a1;
+    uint4 u1h, u1l, u2h, u2l;
+  };
+  auto fetch = [&](int kb) {
+    Operands o;
+    o.a0 = ya[(32 * kb + col) * 4 + g];
+    o.a1 = ya[(32 * kb + 16 + col) * 4 + g];
+    o.u1h = fr[(kb * 2 + 0) * 4 * kSweMfR1];
+    o.u1l = fr[(kb * 2 + 1) * 4 * kSweMfR1];
+    o.u2h = fr2[(kb * 2 + 0) * 4 * kSweMfR2];
+    o.u2l = fr2[(kb * 2 + 1) * 4 * kSweMfR2];
+    return o;
+  };
+  Operands next = fetch(kb0);
 #pragma unroll 1
   for (int kb = kb0; kb < kb1; ++kb) {
-    const float a0 = ya[(32 * kb + col) * 4 + g];
-    const float a1 = ya[(32 * kb + 16 + col) * 4 + g];
-    const swe_mh8 A1h = __builtin_bit_cast(swe_mh8, fr[(kb * 2 + 0) * 4 * kSweMfR1]);
-    const swe_mh8 A1l = __builtin_bit_cast(swe_mh8, fr[(kb * 2 + 1) * 4 * kSweMfR1]);
-    const swe_mh8 A2h = __builtin_bit_cast(swe_mh8, fr2[(kb * 2 + 0) * 4 * kSweMfR2]);
-    const swe_mh8 A2l = __builtin_bit_cast(swe_mh8, fr2[(kb * 2 + 1) * 4 * kSweMfR2]);
+    const Operands cur = next;
+    next = fetch(min(kb + 1, kb1 - 1));
+    const float a0 = cur.a0, a1 = cur.a1;
+    const swe_mh8 A1h = __builtin_bit_cast(swe_mh8, cur.u1h);
+    const swe_mh8 A1l = __builtin_bit_cast(swe_mh8, cur.u1l);
+    const swe_mh8 A2h = __builtin_bit_cast(swe_mh8, cur.u2h);
+    const swe_mh8 A2l = __builtin_bit_cast(swe_mh8, cur.u2l);
     swe_mf4 O[NG][2];
 #pragma unroll
     for (int G = 0; G < NG; ++G) {
@@ -1379,27 +1395,24 @@ __device__ __forceinline__ void swe_mf_add_far(SweAcc& acc, const double* R,
 
 // First pass: the far tiles, and the far sub-tiles of the others, of each
 // wave in source chunk `chunk` of C equal runs of tiles; the 18 raw far sums
-// go to rows 18 row .. of sg.part, added to what they hold if `add`.  The
-// block copies each tile's record to LDS through registers, one tile ahead,
-// into the other of two buffers (buf).  Every thread of the 256 calls it.
+// go to rows 18 row .. of sg.part, added to what they hold if `add`.  Each wave
+// reads the records of its far tiles from L2 and waits for no other.
 //
 // What bounds it: per 64 pairs 37 cycles of vector issue (reciprocal 8, f16
 // splits of w and w^2 16, products 2, the rest once per tile) and 20 of matrix
-// products; at 256 registers two waves of a SIMD overlap little of them (62 %
-// and 32 % busy).  Level 6 (1.0e10 pairs): 3.9 ms, against 4.3 with each wave
-// reading the records from L2, whose loads the compiler would not keep ahead,
-// and one block for all sources of its targets.
+// products; at 256 registers two waves of a SIMD overlap little of them (68 %
+// and 33 % busy).  Level 6 (1.0e10 pairs): 3.76 ms.  Records staged in LDS by
+// the block, a tile ahead, took 3.83 there, and 1.18 ms against 0.85 for eight
+// members of 10,700 cubed-sphere faces, most of whose tiles are near: the block
+// then copies every record and waits for its slowest wave at each.
 template <int BLOCK>
 __device__ __forceinline__ void swe_mf_far_block(
     const SweMfTiles& mt, int nsrc, const SweSeg& sg, int blk, int chunk, int C,
-    const SweParams& P, int row, bool add, uint4 (*buf)[kSweMfRec]) {
-  static_assert(BLOCK == 256, "a thread copies every 256th part of a record");
-  constexpr int kCopy = (kSweMfRec + BLOCK - 1) / BLOCK;
+    const SweParams& P, int row, bool add) {
   const int64_t n_live = sg.d_n ? *sg.d_n : sg.n;
-  if (static_cast<int64_t>(blk) * BLOCK >= n_live) return;
   const int64_t c = static_cast<int64_t>(blk) * BLOCK + threadIdx.x;
+  if (c - (threadIdx.x & 63) >= n_live) return;  // no target in the wave
   const bool in = c < n_live;
-  const bool live = c - (threadIdx.x & 63) < n_live;  // a target in the wave
   const int64_t i = swe_target(sg, c, in);
   const double* px = sg.x + i * sg.es;
   const double x[3] = {px[0], px[sg.cs], px[2 * sg.cs]};
@@ -1408,44 +1421,26 @@ __device__ __forceinline__ void swe_mf_far_block(
   const int ntile = (nsrc + kSweTile - 1) / kSweTile;
   const int t0 = static_cast<int>(static_cast<int64_t>(ntile) * chunk / C);
   const int t1 = static_cast<int>(static_cast<int64_t>(ntile) * (chunk + 1) / C);
-  uint4 ahead[kCopy];
-  auto fetch = [&](int t) {
-    const uint4* p = mt.rec + kSweMfRec * static_cast<int64_t>(t);
-#pragma unroll
-    for (int q = 0; q < kCopy; ++q)
-      ahead[q] = p[min(static_cast<int>(threadIdx.x) + BLOCK * q, kSweMfRec - 1)];
-  };
-  auto store = [&](int b) {
-#pragma unroll
-    for (int q = 0; q < kCopy; ++q)
-      if (static_cast<int>(threadIdx.x) + BLOCK * q < kSweMfRec)
-        buf[b][threadIdx.x + BLOCK * q] = ahead[q];
-  };
   double F1[4][4], F2[4][4];
 #pragma unroll
   for (int G = 0; G < 4; ++G)
 #pragma unroll
     for (int v = 0; v < 4; ++v) F1[G][v] = F2[G][v] = 0.0;
   if (t0 < t1) {
-    fetch(t0);
-    __syncthreads();  // an earlier chunk's last tile is read
-    store(0);
-    __syncthreads();
     double4 cc_next = vload(mt.cen, t0);
-    int b = 0;
 #pragma unroll 1
     for (int t = t0; t < t1; ++t) {
       const double4 cc = cc_next;
       cc_next = vload(mt.cen, min(t + 1, t1 - 1));
-      fetch(min(t + 1, t1 - 1));
+      const uint4* rec = mt.rec + kSweMfRec * static_cast<int64_t>(t);
       // a far tile is one range of k-blocks; a near tile, its far sub-tiles
       // with offsets from their own centroids
       const bool tile_far = !__ballot(in && swe_mf_near(x, cc));
-      const int nrange = !live ? 0 : tile_far ? 1 : kSweMfNsub;
+      const int nrange = tile_far ? 1 : kSweMfNsub;
 #pragma unroll 1
       for (int sub = 0; sub < nrange; ++sub) {
         double4 cs = cc;
-        const uint4* ya = buf[b];
+        const uint4* ya = rec;
         int kb0 = 0, kb1 = kSweMfKb;
         if (!tile_far) {
           cs = mt.scen[kSweMfNsub * static_cast<int64_t>(t) + sub];
@@ -1455,13 +1450,10 @@ __device__ __forceinline__ void swe_mf_far_block(
           kb1 = kb0 + kSweMfSub / 32;
         }
         const double e0 = x[0] - cs.x, e1 = x[1] - cs.y, e2 = x[2] - cs.z;
-        swe_mf_far_tile(buf[b], reinterpret_cast<const float*>(ya), kb0, kb1, in,
+        swe_mf_far_tile(rec, reinterpret_cast<const float*>(ya), kb0, kb1, in,
                         e0, e1, e2, e0 * e0 + e1 * e1 + e2 * e2, cs.w, P.eps2,
                         col, g, F1, F2);
       }
-      b ^= 1;
-      store(b);  // every wave passed its last read of this buffer one tile ago
-      __syncthreads();
     }
   }
   double R[kSweMfRows];
@@ -1586,7 +1578,6 @@ template <int BLOCK, int MINW>
 __global__ __launch_bounds__(BLOCK, MINW) void swe_mf_far_kernel(
     const SweSrc* __restrict__, const double4* __restrict__,
     const int32_t* __restrict__ count, SweSeg s0, SweSeg s1, SweParams P) {
-  __shared__ uint4 buf[2][kSweMfRec];
   const int b = flat_block() / P.rows;
   const int k0 = flat_block() % P.rows;
   const bool first = b < s0.nblocks;
@@ -1594,7 +1585,7 @@ __global__ __launch_bounds__(BLOCK, MINW) void swe_mf_far_kernel(
   const int blk = first ? b : b - s0.nblocks;
 #pragma unroll 1
   for (int k = k0; k < P.C; k += P.rows)
-    swe_mf_far_block<BLOCK>(P.mf, *count, sg, blk, k, P.C, P, k0, k != k0, buf);
+    swe_mf_far_block<BLOCK>(P.mf, *count, sg, blk, k, P.C, P, k0, k != k0);
 }
 
 // SHARE: pairs per FP64 reciprocal in near sub-tiles (2 or 4).
@@ -1819,7 +1810,6 @@ __device__ __forceinline__ void swe_ens_far(SweSeg& sg, const EnsMember& M,
 template <int BLOCK, int MINW>
 __global__ __launch_bounds__(BLOCK, MINW) void swe_ens_mf_far_kernel(
     SweEnsArgs A, double* part) {
-  __shared__ uint4 buf[2][kSweMfRec];
   if (flat_block() >= A.n_items) return;
   const int4 w = A.items[flat_block()];
   const EnsMember M = A.mem[w.x];
@@ -1830,7 +1820,7 @@ __global__ __launch_bounds__(BLOCK, MINW) void swe_ens_mf_far_kernel(
 #pragma unroll 1
   for (int k = w.w; k < M.C; k += step)
     swe_mf_far_block<BLOCK>(mt, M.cnt, sg, w.z, k, M.C, A.P,
-                            A.P.rows == 1 ? 0 : k, k != w.w, buf);
+                            A.P.rows == 1 ? 0 : k, k != w.w);
 }
 
 template <int MINW, int SHARE>
